@@ -696,15 +696,15 @@ def bench_ops(nr, args):
             "ops": res}
 
 
-VALU_F32_PEAK_TFLOPS = 78.6  # 256 CUs x 4 SIMDs x 16 lanes x 2 flops x 2.4 GHz, one v_fma_f32 per lane
+MFMA_F32_PEAK_TFLOPS = 157.3  # 256 CUs x 4 SIMDs x 64 flops per cycle x 2.4 GHz (v_mfma_f32_32x32x2_f32: 4096 in 64)
 
 
 def bench_matmul(nr, args):
     """nt_hip_matmul (GpuBackend::matmul, CpuRef's fma-chain order bit for bit) at the reference's
     matmul_throughput shapes (src/tensor/tests/gpu/kernels.rs:262-291: A.B 1024^3, A.B 512x512x2048,
-    A.B^T 512x2048x512, A^T.B 512x512x2048) and at 4096^3, on resident f32 operands. The order
-    rules out the matrix cores, so the roofline is the VALU's f32 fma rate without packed
-    instructions (78.6 TFLOP/s)."""
+    A.B^T 512x2048x512, A^T.B 512x512x2048) and at 4096^3, on resident f32 operands. The f32
+    MFMA instructions add their products in that order, so the roofline is their rate (157.3
+    TFLOP/s)."""
     from noetic_ops import Layout
     L = nr.lib()
     P = lambda t: C.c_void_p(t.ptr)  # noqa: E731
@@ -724,7 +724,7 @@ def bench_matmul(nr, args):
         ck = lambda rc: nr._check(rc, "matmul")  # noqa: E731
         ms, _ = timed(nr, steps, warmup, lambda i: ck(L.nt_hip_matmul(P(a), C.byref(ca), P(b), C.byref(cb), P(y))))
         tf = 2.0 * m * k * n / (ms * 1e-3) / 1e12
-        res[name] = {"ms": round(ms, 4), "tflops": round(tf, 2), "frac_of_valu_peak": round(tf / VALU_F32_PEAK_TFLOPS, 4)}
+        res[name] = {"ms": round(ms, 4), "tflops": round(tf, 2), "frac_of_f32_mfma_peak": round(tf / MFMA_F32_PEAK_TFLOPS, 4)}
         if name in ("A.B 1024^3", "A.B 4096^3"):
             ms, _ = timed(nr, steps, warmup,
                           lambda i: ck(L.nt_hip_matmul_half(P(a), C.byref(ca), P(b), C.byref(cb), P(y))))
@@ -738,10 +738,10 @@ def bench_matmul(nr, args):
            "dtype": "f32", "data": "synthetic",
            "config": {"workload": "matmul: uniform(-2, 2) f32 operands resident on the device, fresh-output-free "
                                   "(one preallocated output per shape)"},
-           "roofline": {"bound": "valu", "achieved": top["tflops"], "peak": VALU_F32_PEAK_TFLOPS, "unit": "TFLOP/s",
-                        "frac": top["frac_of_valu_peak"], "traffic": None,
-                        "note": "the published 157.3 TFLOP/s f32 figure counts matrix-core or packed-f32 "
-                                "instructions; neither keeps the reference's per-output fma chain"},
+           "roofline": {"bound": "mfma", "achieved": top["tflops"], "peak": MFMA_F32_PEAK_TFLOPS, "unit": "TFLOP/s",
+                        "frac": top["frac_of_f32_mfma_peak"], "traffic": None,
+                        "note": "v_mfma_f32_32x32x2_f32 over ascending k is the reference's per-output fma "
+                                "chain, bit for bit"},
            "shapes": res}
     if args.cpu_rows > 0:
         import time as _t

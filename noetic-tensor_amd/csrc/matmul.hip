@@ -2,18 +2,27 @@
 // bit for bit the reference's product. The reference fixes the arithmetic of every output
 // (src/tensor/cuda/kernels.rs:14-20, the order of matrixmultiply 0.3.11's sgemm that CpuRef calls
 // per batch, src/tensor/kernels.rs:415-420): an fma chain from zero over k in order, closed every
-// 256 k; the first block's chain is the total and each later block's chain is added to it. That
-// order allows no split of one output's chain over lanes and no matrix-core instruction (an MFMA
-// sums several products before it rounds), so this is a VALU kernel: each of a block's 256
-// threads owns an 8x8 (or 4x4) register tile of outputs and runs their 64 (16) chains side by
-// side, one v_fma_f32 per product, on A and B panels staged through LDS.
+// 256 k; the first block's chain is the total and each later block's chain is added to it.
 //
-// Layout of a 128x128 block tile: thread (tx, ty) = (tid % 16, tid / 16) owns rows
-// {ty*4 + i, 64 + ty*4 + i} and columns {tx*4 + j, 64 + tx*4 + j} (i, j < 4), so each k step
-// reads its 8 A values and 8 B values as four 16-byte LDS reads (A's are broadcast: a wave spans
-// four ty). The panels are double-buffered (one barrier per 16 k). Workgroups are renumbered so
-// that each of the 8 XCDs (which the hardware deals consecutive workgroups to in turn) works on a
-// contiguous run of tiles, whose A panels then stay in that XCD's L2.
+// The chains run on the matrix cores. On gfx950 v_mfma_f32_32x32x2_f32 adds its two products one
+// after the other, each with one rounding, subnormals kept: the bits of
+// fma(a1, b1, fma(a0, b0, c)) (tests/test_matmul_mfma_gpu.py compares them on normal, subnormal,
+// cancelling, overflowing and special operands). So a run of them over ascending k is the
+// reference's chain, at twice the rate of v_fma_f32 (157.3 against 78.6 TFLOP/s nominal).
+//
+// A workgroup computes a 128x128 (eight waves of 2 x 1 MFMA tiles) or 64x64 (four waves of one) tile;
+// panels of 32 k go through LDS, double-buffered, one barrier per panel.
+// LDS holds 32 k of a row (of A) or column (of B) with each 8 k as [0 2 4 6 | 1 3 5 7]: an MFMA's
+// lanes 0-31 take its first k and lanes 32-63 its second, so one 16-byte read per lane holds four
+// MFMAs' operands. Rows are 36 words apart: the reads are free of bank conflicts. A panel of 128 x
+// 128 costs a wave 12 such reads against 32 MFMAs of 64 cycles, so what bounds a large product is
+// the matrix cores' rate: 4096^3 takes 1118 us (123 TFLOP/s; the VALU kernel before it 1920 us, 71.6),
+// 2048^3 142 us (251), 1024^3 27.7 us (50.0). Past the last k both operands are padded with -0 and +0, whose product
+// -0 leaves every sum as it is (+0 would turn a chain's -0 into +0).
+//
+// Workgroups are renumbered so that each of the 8 XCDs (which the hardware deals consecutive
+// workgroups to in turn) works on a contiguous run of tiles, whose A panels then stay in that
+// XCD's L2.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -36,10 +45,10 @@ namespace nt {
 namespace {
 
 constexpr int kMmThreads = 256;
-constexpr int kBK = 16;    // k per LDS stage
+constexpr int kBK = 32;    // k per LDS panel
 constexpr int kKC = 256;   // the chain is closed every kKC k
 constexpr int kMaxBatchDims = NT_MAX_RANK - 2;
-constexpr int kPad = 4;    // LDS row padding (keeps 16-byte alignment, spreads the stores' banks)
+constexpr int kLdsRow = kBK + 4;  // words between LDS rows
 
 struct MatmulP {
     const float *a, *b;
@@ -59,39 +68,75 @@ struct MatmulP {
     int32_t avec, bvec;            // matmul_half: the operand may be staged with 16-byte loads
 };
 
-// H = 2: 128x128 tile, 8x8 outputs per thread; H = 1: 64x64 tile, 4x4 per thread.
-// AK: A is read along k (a_cs == 1); otherwise along m. BN: B is read along n (b_cs == 1);
-// otherwise along k. Either way consecutive lanes read consecutive addresses when the view is
-// contiguous along that dimension.
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+// (16-byte loads of elements that are only 4-byte aligned, as rows of an odd length start)
+typedef f32x4_t f32x4_any __attribute__((aligned(4)));
+
+// Eight elements k .. k + 7 of one row of A (column of B) at src, `stride` apart (K1: adjacent), into
+// two vectors in order: what reorders them waits for the loads, so that is left to the store into LDS.
+template <bool K1>
+__device__ __forceinline__ void load8(const float *src, int64_t stride, f32x4_t (&x)[2]) {
+    if constexpr (K1) {
+        x[0] = reinterpret_cast<const f32x4_any *>(src)[0];
+        x[1] = reinterpret_cast<const f32x4_any *>(src)[1];
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++) x[e / 4][e % 4] = src[e * stride];
+    }
+}
+
+// The same of the last panel, when K does not end with it: elements at or past `lim` are `pad`.
+__device__ __forceinline__ void load8_tail(const float *src, int64_t stride, int lim, float pad, f32x4_t (&x)[2]) {
+#pragma unroll
+    for (int e = 0; e < 8; e++) x[e / 4][e % 4] = e < lim ? src[e * stride] : pad;
+}
+
+// A tile of NM x NN waves, each WM x WN MFMA tiles of 32 x 32. Two waves per SIMD (eight per 128 x 128
+// tile) let one's MFMAs cover the other's waits: 4096^3 in 1118 us (123 TFLOP/s, 78% of the matrix
+// cores' 157.3) against 1202 with four waves of 2 x 2 MFMA tiles; 256 x 128 tiles took 1152.
+template <int WM_, int WN_, int NM_, int NN_>
+struct MmTile {
+    static constexpr int WM = WM_, WN = WN_, NM = NM_, NN = NN_;
+    static constexpr int kTM = 32 * WM * NM, kTN = 32 * WN * NN, kThreads = 64 * NM * NN;
+};
+using Tile64 = MmTile<1, 1, 2, 2>;     // 64 x 64, 256 threads
+using Tile128 = MmTile<2, 1, 2, 4>;    // 128 x 128, 512 threads
+
+// AK: A is contiguous along k (a_cs == 1): a thread loads 8 k of a row as two 16-byte loads, four
+// threads a row of the panel. Otherwise a wave's lanes take consecutive rows, a load for each k.
+// BN: a wave's lanes take consecutive columns of B; otherwise B is contiguous along k (b_rs == 1) and
+// loaded as A is. Consecutive lanes read consecutive addresses when the view is contiguous along
+// either dimension.
 // SPLIT: the workgroup covers kc_per 256-k blocks of its tile and writes each block's chain to
 // that block's slice; k_fold then closes the chains in order (the same arithmetic, more
 // workgroups for outputs too few to fill the chip).
-template <int H, bool AK, bool BN, bool SPLIT>
-__device__ __forceinline__ void matmul_body(const MatmulP &p) {
-    constexpr int T = 64 * H;             // tile edge
-    constexpr int LPT = T * kBK / kMmThreads;  // elements of each panel a thread loads per stage
-    __shared__ __attribute__((aligned(16))) float As[2][kBK][T + kPad];
-    __shared__ __attribute__((aligned(16))) float Bs[2][kBK][T + kPad];
+template <class C, bool AK, bool BN, bool SPLIT>
+__global__ __launch_bounds__(C::kThreads, 2) void k_matmul(MatmulP p) {
+    constexpr int WM = C::WM, WN = C::WN, TM = C::kTM, TN = C::kTN, kThreads = C::kThreads;
+    // groups of 8 k each thread stages per panel
+    constexpr int GA = TM * kBK / 8 / kThreads, GB = TN * kBK / 8 / kThreads;
+    __shared__ __attribute__((aligned(16))) float As[2][TM * kLdsRow];
+    __shared__ __attribute__((aligned(16))) float Bs[2][TN * kLdsRow];
 
-    const int tid = threadIdx.x;
-    const int tx = tid % 16, ty = tid / 16;
+    const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
     int64_t wg = blockIdx.x;
     const int64_t full = p.blocks / 8 * 8;
     if (wg < full) wg = (wg % 8) * (full / 8) + wg / 8;
     const int64_t per_batch = int64_t(p.tm) * p.tn;
-    int64_t zs = wg / per_batch;  // split * batches + batch
-    const int64_t rem = wg - zs * per_batch;
+    int64_t z = wg / per_batch;  // split * batches + batch
+    const int64_t rem = wg - z * per_batch;
     int kbeg = 0, kend = p.k;
     if constexpr (SPLIT) {
         int64_t nbat = 1;
         for (int d = 0; d < p.nbd; d++) nbat *= p.bshape[d];
-        const int sp = int(zs / nbat);
-        zs -= int64_t(sp) * nbat;
+        const int sp = int(z / nbat);
+        z -= int64_t(sp) * nbat;
         kbeg = sp * p.kc_per * kKC;
         kend = min(p.k, kbeg + p.kc_per * kKC);
     }
-    const int64_t z = zs;
-    const int row0 = int(rem / p.tn) * T, col0 = int(rem % p.tn) * T;
+    const int row0 = int(rem / p.tn) * TM, col0 = int(rem % p.tn) * TN;
     int64_t ao = p.a_off, bo = p.b_off;
     {
         int64_t q = z;
@@ -102,240 +147,174 @@ __device__ __forceinline__ void matmul_body(const MatmulP &p) {
             bo += i * p.b_bs[d];
         }
     }
-    const float *a = p.a + ao;
-    const float *b = p.b + bo;
     const int M = p.m, N = p.n, K = p.k;
 
-    float ra[LPT], rb[LPT];
-    // Interior panels of a view contiguous along one axis (16-byte aligned) load four values per
-    // instruction. Along k (A row-major, B transposed): group g is row or column g / 4, k (g % 4) * 4
-    // .. + 3. Along m or n (A transposed, B row-major): group g is k g / (T / 4), rows or columns
-    // (g % (T / 4)) * 4 .. + 3.
-    constexpr int V4 = LPT / 4;
-    auto vec_a = [&](int k0) { return p.avec && row0 + T <= M && k0 + kBK <= K; };
-    auto vec_b = [&](int k0) { return p.bvec && col0 + T <= N && k0 + kBK <= K; };
+    // This thread's groups: their row (column) in the tile, first k in the panel, LDS offset and
+    // source. A row past the last one reads row 0 (its outputs are not stored).
+    const float *asrc[GA], *bsrc[GB];
+    int akg[GA], bkg[GB], alds[GA], blds[GB];
+#pragma unroll
+    for (int q = 0; q < GA; q++) {
+        const int g = tid + kThreads * q, r = AK ? g / (kBK / 8) : g % TM;
+        akg[q] = 8 * (AK ? g % (kBK / 8) : g / TM);
+        alds[q] = r * kLdsRow + akg[q];
+        asrc[q] = p.a + ao + int64_t(row0 + r < M ? row0 + r : 0) * p.a_rs + int64_t(akg[q]) * p.a_cs;
+    }
+#pragma unroll
+    for (int q = 0; q < GB; q++) {
+        const int g = tid + kThreads * q, c = BN ? g % TN : g / (kBK / 8);
+        bkg[q] = 8 * (BN ? g / TN : g % (kBK / 8));
+        blds[q] = c * kLdsRow + bkg[q];
+        bsrc[q] = p.b + bo + int64_t(col0 + c < N ? col0 + c : 0) * p.b_cs + int64_t(bkg[q]) * p.b_rs;
+    }
+    f32x4_t ra[GA][2], rb[GB][2];
     auto load = [&](int k0) {
-        const bool va = vec_a(k0), vb = vec_b(k0);
-        if (va) {
 #pragma unroll
-            for (int q = 0; q < V4; q++) {
-                const int g = tid + kMmThreads * q;
-                const float *src = AK ? a + int64_t(row0 + g / 4) * p.a_rs + k0 + (g % 4) * 4
-                                      : a + int64_t(k0 + g / (T / 4)) * p.a_cs + row0 + (g % (T / 4)) * 4;
-                const float4 v = *reinterpret_cast<const float4 *>(src);
-                ra[4 * q] = v.x;
-                ra[4 * q + 1] = v.y;
-                ra[4 * q + 2] = v.z;
-                ra[4 * q + 3] = v.w;
-            }
-        }
-        if (vb) {
+        for (int q = 0; q < GA; q++) load8<AK>(asrc[q] + int64_t(k0) * p.a_cs, p.a_cs, ra[q]);
 #pragma unroll
-            for (int q = 0; q < V4; q++) {
-                const int g = tid + kMmThreads * q;
-                const float *src = BN ? b + int64_t(k0 + g / (T / 4)) * p.b_rs + col0 + (g % (T / 4)) * 4
-                                      : b + int64_t(col0 + g / 4) * p.b_cs + k0 + (g % 4) * 4;
-                const float4 v = *reinterpret_cast<const float4 *>(src);
-                rb[4 * q] = v.x;
-                rb[4 * q + 1] = v.y;
-                rb[4 * q + 2] = v.z;
-                rb[4 * q + 3] = v.w;
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < LPT; i++) {
-            const int e = tid + kMmThreads * i;
-            int r, kk;
-            if constexpr (AK) {
-                kk = e % kBK;
-                r = e / kBK;
-            } else {
-                r = e % T;
-                kk = e / T;
-            }
-            const int gr = row0 + r, gk = k0 + kk;
-            if (!va) ra[i] = (gr < M && gk < K) ? a[int64_t(gr) * p.a_rs + int64_t(gk) * p.a_cs] : 0.0f;
-            int cc;
-            if constexpr (BN) {
-                cc = e % T;
-                kk = e / T;
-            } else {
-                kk = e % kBK;
-                cc = e / kBK;
-            }
-            const int gc = col0 + cc, gk2 = k0 + kk;
-            if (!vb) rb[i] = (gc < N && gk2 < K) ? b[int64_t(gk2) * p.b_rs + int64_t(gc) * p.b_cs] : 0.0f;
-        }
+        for (int q = 0; q < GB; q++) load8<!BN>(bsrc[q] + int64_t(k0) * p.b_rs, p.b_rs, rb[q]);
     };
-    auto stash = [&](int s, int k0) {
-        if (vec_a(k0)) {
+    auto put8 = [&](float *d, const f32x4_t(&x)[2]) {
+        reinterpret_cast<f32x4_t *>(d)[0] = f32x4_t{x[0][0], x[0][2], x[1][0], x[1][2]};
+        reinterpret_cast<f32x4_t *>(d)[1] = f32x4_t{x[0][1], x[0][3], x[1][1], x[1][3]};
+    };
+    auto stash = [&](int s) {
 #pragma unroll
-            for (int q = 0; q < V4; q++) {
-                const int g = tid + kMmThreads * q;
-                if constexpr (AK) {
+        for (int q = 0; q < GA; q++) put8(&As[s][alds[q]], ra[q]);
 #pragma unroll
-                    for (int j = 0; j < 4; j++) As[s][(g % 4) * 4 + j][g / 4] = ra[4 * q + j];
-                } else {
-                    *reinterpret_cast<float4 *>(&As[s][g / (T / 4)][(g % (T / 4)) * 4]) =
-                        make_float4(ra[4 * q], ra[4 * q + 1], ra[4 * q + 2], ra[4 * q + 3]);
-                }
-            }
-        } else {
+        for (int q = 0; q < GB; q++) put8(&Bs[s][blds[q]], rb[q]);
+    };
+
+    // The wave's part: rows wr .. wr + 32 WM - 1, columns wc .. wc + 32 WN - 1 of the tile.
+    const int wr = (wave / C::NN) * 32 * WM, wc = (wave % C::NN) * 32 * WN;
+    const int aread = (wr + lane % 32) * kLdsRow + 4 * (lane / 32);
+    const int bread = (wc + lane % 32) * kLdsRow + 4 * (lane / 32);
+    f32x16_t acc[WM][WN], tot[SPLIT ? 1 : WM][SPLIT ? 1 : WN];
+    auto clear = [&]() {
 #pragma unroll
-            for (int i = 0; i < LPT; i++) {
-                const int e = tid + kMmThreads * i;
-                if constexpr (AK) As[s][e % kBK][e / kBK] = ra[i];
-                else As[s][e / T][e % T] = ra[i];
-            }
-        }
-        if (vec_b(k0)) {
+        for (int i = 0; i < WM; i++)
 #pragma unroll
-            for (int q = 0; q < V4; q++) {
-                const int g = tid + kMmThreads * q;
-                if constexpr (BN) {
-                    *reinterpret_cast<float4 *>(&Bs[s][g / (T / 4)][(g % (T / 4)) * 4]) =
-                        make_float4(rb[4 * q], rb[4 * q + 1], rb[4 * q + 2], rb[4 * q + 3]);
-                } else {
+            for (int j = 0; j < WN; j++)
 #pragma unroll
-                    for (int j = 0; j < 4; j++) Bs[s][(g % 4) * 4 + j][g / 4] = rb[4 * q + j];
-                }
-            }
-        } else {
+                for (int v = 0; v < 16; v++) acc[i][j][v] = 0.0f;
+    };
+    clear();
+    f32x4_t fa[2][WM], fb[2][WN];  // two groups' operands: one in use, the next on its way from LDS
+    auto fetch = [&](int s, int kg) {  // k 8 kg .. 8 kg + 7 of the panel
 #pragma unroll
-            for (int i = 0; i < LPT; i++) {
-                const int e = tid + kMmThreads * i;
-                if constexpr (BN) Bs[s][e / T][e % T] = rb[i];
-                else Bs[s][e % kBK][e / kBK] = rb[i];
-            }
+        for (int i = 0; i < WM; i++)
+            fa[kg % 2][i] = *reinterpret_cast<const f32x4_t *>(&As[s][aread + 32 * i * kLdsRow + 8 * kg]);
+#pragma unroll
+        for (int j = 0; j < WN; j++)
+            fb[kg % 2][j] = *reinterpret_cast<const f32x4_t *>(&Bs[s][bread + 32 * j * kLdsRow + 8 * kg]);
+    };
+    auto group = [&](int kg) {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int i = 0; i < WM; i++)
+#pragma unroll
+                for (int j = 0; j < WN; j++)
+                    acc[i][j] =
+                        __builtin_amdgcn_mfma_f32_32x32x2f32(fa[kg % 2][i][e], fb[kg % 2][j][e], acc[i][j], 0, 0, 0);
+    };
+    // Lane l's value v of MFMA tile (i, j): row wr + 32 i + 8 (v / 4) + 4 (l / 32) + v % 4, column
+    // wc + 32 j + l % 32: a store instruction writes 32 consecutive columns of two rows.
+    auto put = [&](float *c, const f32x16_t &t, int i, int j) {
+        const int col = col0 + wc + 32 * j + lane % 32;
+        if (col >= N) return;
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            const int row = row0 + wr + 32 * i + 8 * (v / 4) + 4 * (lane / 32) + v % 4;
+            if (row < M) c[int64_t(row) * N + col] = t[v];
         }
     };
 
-    float acc[4 * H][4 * H], tot[SPLIT ? 1 : 4 * H][SPLIT ? 1 : 4 * H];
+    auto close = [&](int k0) {  // the chain of the 256-k block that k0 lies in ends
+        if constexpr (SPLIT) {
 #pragma unroll
-    for (int i = 0; i < 4 * H; i++)
+            for (int i = 0; i < WM; i++)
 #pragma unroll
-        for (int j = 0; j < 4 * H; j++) acc[i][j] = 0.0f;
+                for (int j = 0; j < WN; j++)
+                    put(p.slices + int64_t(k0 / kKC) * p.outputs + z * int64_t(M) * N, acc[i][j], i, j);
+        } else {
+            const bool first = k0 < kKC;
+#pragma unroll
+            for (int i = 0; i < WM; i++)
+#pragma unroll
+                for (int j = 0; j < WN; j++)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) tot[i][j][v] = first ? acc[i][j][v] : acc[i][j][v] + tot[i][j][v];
+        }
+        clear();
+    };
+
+    // The whole panels. Panel i's iteration finds its group 0 in registers and the panel whole in LDS
+    // buffer s. The next panel is written to the other buffer (last read before the previous
+    // barrier) ahead of group 2, and the barrier comes between groups 2 and 3, so that group 3's
+    // MFMAs cover the next panel's first reads; the panel after it is loaded meanwhile. (No branch:
+    // the last iterations load and store the last panel once more.)
+    static_assert(kBK == 32, "four groups of 8 k per panel");
+    const int kfull = kbeg + (kend - kbeg) / kBK * kBK, klast = kfull - kBK;
+    if (kbeg < kfull) {
+        load(kbeg);
+        stash(0);
+        load(min(kbeg + kBK, klast));
+        __syncthreads();
+        fetch(0, 0);
+        int s = 0;
+        for (int k0 = kbeg; k0 < kfull; k0 += kBK) {
+            fetch(s, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            group(0);
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(s, 2);
+            __builtin_amdgcn_sched_barrier(0);
+            group(1);
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(s, 3);
+            stash(s ^ 1);
+            load(min(k0 + 2 * kBK, klast));
+            __builtin_amdgcn_sched_barrier(0);
+            group(2);
+            __builtin_amdgcn_sched_barrier(0);
+            __syncthreads();
+            fetch(s ^ 1, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            group(3);
+            __builtin_amdgcn_sched_barrier(0);
+            if ((k0 + kBK) % kKC == 0 || k0 + kBK == kend) close(k0);
+            s ^= 1;
+        }
+    }
+    if (kfull < kend) {  // the last panel, when K ends inside it
+#pragma unroll
+        for (int q = 0; q < GA; q++)
+            load8_tail(asrc[q] + int64_t(kfull) * p.a_cs, p.a_cs, K - kfull - akg[q], -0.0f, ra[q]);
+#pragma unroll
+        for (int q = 0; q < GB; q++)
+            load8_tail(bsrc[q] + int64_t(kfull) * p.b_rs, p.b_rs, K - kfull - bkg[q], 0.0f, rb[q]);
+        __syncthreads();  // (the reads of the last whole panel are done)
+        stash(0);
+        __syncthreads();
+#pragma unroll
+        for (int kg = 0; kg < kBK / 8; kg++) {
+            fetch(0, kg);
+            group(kg);
+        }
+        close(kfull);
+    }
     if constexpr (!SPLIT) {
 #pragma unroll
-        for (int i = 0; i < 4 * H; i++)
+        for (int i = 0; i < WM; i++)
 #pragma unroll
-            for (int j = 0; j < 4 * H; j++) tot[i][j] = 0.0f;
+            for (int j = 0; j < WN; j++) {
+                if (K == 0)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) tot[i][j][v] = 0.0f;
+                put(p.c + z * int64_t(M) * N, tot[i][j], i, j);
+            }
     }
-    // split-k: a closed chain goes to its 256-k block's slice, at the tile's outputs
-    auto put_slice = [&](int kc) {
-        float *sl = p.slices + int64_t(kc) * p.outputs + z * int64_t(p.m) * p.n;
-#pragma unroll
-        for (int hr = 0; hr < H; hr++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int r = row0 + hr * 64 + ty * 4 + i;
-                if (r >= p.m) continue;
-#pragma unroll
-                for (int hc = 0; hc < H; hc++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const int cc = col0 + hc * 64 + tx * 4 + j;
-                        if (cc < p.n) sl[int64_t(r) * p.n + cc] = acc[hr * 4 + i][hc * 4 + j];
-                    }
-            }
-    };
-
-    auto step = [&](int s, int kk) {
-        float av[4 * H], bv[4 * H];
-#pragma unroll
-        for (int h = 0; h < H; h++) {
-            const float4 x = *reinterpret_cast<const float4 *>(&As[s][kk][h * 64 + ty * 4]);
-            const float4 y = *reinterpret_cast<const float4 *>(&Bs[s][kk][h * 64 + tx * 4]);
-            av[4 * h] = x.x;
-            av[4 * h + 1] = x.y;
-            av[4 * h + 2] = x.z;
-            av[4 * h + 3] = x.w;
-            bv[4 * h] = y.x;
-            bv[4 * h + 1] = y.y;
-            bv[4 * h + 2] = y.z;
-            bv[4 * h + 3] = y.w;
-        }
-#pragma unroll
-        for (int i = 0; i < 4 * H; i++)
-#pragma unroll
-            for (int j = 0; j < 4 * H; j++) acc[i][j] = fmaf(av[i], bv[j], acc[i][j]);
-    };
-
-    load(kbeg);
-    stash(0, kbeg);
-    __syncthreads();
-    int s = 0;
-    for (int k0 = kbeg; k0 < kend; k0 += kBK) {
-        const bool more = k0 + kBK < kend;
-        if (more) load(k0 + kBK);  // the next panels' loads are in flight during this stage
-        if (k0 + kBK <= K) {
-#pragma unroll
-            for (int kk = 0; kk < kBK; kk++) step(s, kk);
-        } else {
-            const int kmax = K - k0;
-            for (int kk = 0; kk < kmax; kk++) step(s, kk);
-        }
-        if ((k0 + kBK) % kKC == 0 || !more) {
-            if constexpr (SPLIT) {
-                put_slice(k0 / kKC);
-#pragma unroll
-                for (int i = 0; i < 4 * H; i++)
-#pragma unroll
-                    for (int j = 0; j < 4 * H; j++) acc[i][j] = 0.0f;
-            } else {
-                const bool first = k0 < kKC;
-#pragma unroll
-                for (int i = 0; i < 4 * H; i++)
-#pragma unroll
-                    for (int j = 0; j < 4 * H; j++) {
-                        tot[i][j] = first ? acc[i][j] : acc[i][j] + tot[i][j];
-                        acc[i][j] = 0.0f;
-                    }
-            }
-        }
-        if (more) stash(s ^ 1, k0 + kBK);  // the other buffer was last read before the previous barrier
-        __syncthreads();
-        s ^= 1;
-    }
-    if constexpr (SPLIT) return;
-
-    float *c = p.c + z * int64_t(M) * N;
-    const bool vec = (N % 4) == 0;
-#pragma unroll
-    for (int hr = 0; hr < H; hr++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int r = row0 + hr * 64 + ty * 4 + i;
-            if (r >= M) continue;
-            float *crow = c + int64_t(r) * N;
-#pragma unroll
-            for (int hc = 0; hc < H; hc++) {
-                const int c0 = col0 + hc * 64 + tx * 4;
-                const int ri = SPLIT ? 0 : hr * 4 + i, cj = SPLIT ? 0 : hc * 4;
-                if (vec && c0 + 3 < N) {
-                    *reinterpret_cast<float4 *>(crow + c0) =
-                        make_float4(tot[ri][SPLIT ? 0 : cj], tot[ri][SPLIT ? 0 : cj + 1], tot[ri][SPLIT ? 0 : cj + 2],
-                                    tot[ri][SPLIT ? 0 : cj + 3]);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 4; j++)
-                        if (c0 + j < N) crow[c0 + j] = tot[ri][SPLIT ? 0 : cj + j];
-                }
-            }
-        }
-}
-
-// The 128 tile's 128 accumulators fill the register file at one wave per SIMD; asking for two
-// waves per SIMD spills a few rarely used registers to scratch and lets one wave's fmas cover the
-// other's LDS reads (3.39 -> 2.33 ms at 4096^3). The 64 tile keeps its 4-5 waves per SIMD.
-template <bool AK, bool BN, bool SPLIT>
-__global__ __launch_bounds__(kMmThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_matmul128(MatmulP p) {
-    matmul_body<2, AK, BN, SPLIT>(p);
-}
-
-template <bool AK, bool BN, bool SPLIT>
-__global__ __launch_bounds__(kMmThreads) void k_matmul64(MatmulP p) {
-    matmul_body<1, AK, BN, SPLIT>(p);
 }
 
 // Split-k's closing pass: per output, the first 256-k block's chain is the total and each later
@@ -362,7 +341,6 @@ __global__ void k_fold(const float *slices, int64_t outputs, int nkc, float *out
 // load: along k they go to LDS as they are, along m or n each thread loads a 4x4 block and
 // transposes it in registers, so that every LDS store writes four bf16 of one row.
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
 constexpr int kHPad = 8;  // bf16 padding per LDS row (rows stay 16-byte aligned)
 
 __device__ __forceinline__ uint16_t bf16_bits(float x) {
@@ -740,21 +718,20 @@ __global__ __launch_bounds__(256) void k_half_tiles(MatmulP p, const uint8_t *pa
     }
 }
 
-template <int H, bool SPLIT>
+template <class C, bool SPLIT>
 int launch_matmul(const MatmulP &p, bool ak, bool bn, hipStream_t s) {
-    const dim3 grid(unsigned(p.blocks)), block(kMmThreads);
-    if constexpr (H == 2) {
-        if (ak && bn) hipLaunchKernelGGL((k_matmul128<true, true, SPLIT>), grid, block, 0, s, p);
-        else if (ak) hipLaunchKernelGGL((k_matmul128<true, false, SPLIT>), grid, block, 0, s, p);
-        else if (bn) hipLaunchKernelGGL((k_matmul128<false, true, SPLIT>), grid, block, 0, s, p);
-        else hipLaunchKernelGGL((k_matmul128<false, false, SPLIT>), grid, block, 0, s, p);
-    } else {
-        if (ak && bn) hipLaunchKernelGGL((k_matmul64<true, true, SPLIT>), grid, block, 0, s, p);
-        else if (ak) hipLaunchKernelGGL((k_matmul64<true, false, SPLIT>), grid, block, 0, s, p);
-        else if (bn) hipLaunchKernelGGL((k_matmul64<false, true, SPLIT>), grid, block, 0, s, p);
-        else hipLaunchKernelGGL((k_matmul64<false, false, SPLIT>), grid, block, 0, s, p);
-    }
+    const dim3 grid(unsigned(p.blocks)), block(C::kThreads);
+    if (ak && bn) hipLaunchKernelGGL((k_matmul<C, true, true, SPLIT>), grid, block, 0, s, p);
+    else if (ak) hipLaunchKernelGGL((k_matmul<C, true, false, SPLIT>), grid, block, 0, s, p);
+    else if (bn) hipLaunchKernelGGL((k_matmul<C, false, true, SPLIT>), grid, block, 0, s, p);
+    else hipLaunchKernelGGL((k_matmul<C, false, false, SPLIT>), grid, block, 0, s, p);
     return launched("k_matmul");
+}
+
+template <bool SPLIT>
+int launch_tile(int tile, const MatmulP &p, bool ak, bool bn, hipStream_t s) {
+    if (tile == 128) return launch_matmul<Tile128, SPLIT>(p, ak, bn, s);
+    return launch_matmul<Tile64, SPLIT>(p, ak, bn, s);
 }
 
 }  // namespace
@@ -804,51 +781,44 @@ int nt_hip_matmul(const float *a, const NtLayout *al, const float *b, const NtLa
     p.m = int32_t(m);
     p.n = int32_t(n);
     p.k = int32_t(k);
-    // 128x128 tiles when they give at least two workgroups per CU of the 256, else 64x64.
+    // 128x128 tiles when they give every CU of the 256 a workgroup, else 64x64. Measured (us, 128 /
+    // 64 tiles): 2048^3 (256 tiles of 128) 142 / 161, 1500 x 700 x 1900 (180) 54.3 / 46.9, 1024^3 (64)
+    // 72.7 / 27.7.
     const int64_t big = nb * ((m + 127) / 128) * ((n + 127) / 128);
-    const int H = big >= 512 ? 2 : 1;
-    const int T = 64 * H;
+    const int T = big >= 256 ? 128 : 64;
     p.tm = int32_t((m + T - 1) / T);
     p.tn = int32_t((n + T - 1) / T);
     const int64_t tiles = nb * p.tm * p.tn;
     p.outputs = nb * m * n;
-    // Split k over more workgroups when the tiles alone leave CUs idle: each workgroup takes
-    // kc_per of the ceil(k / 256) chains, so that about 1024 workgroups run in all.
+    // Split k over more workgroups when the tiles alone leave CUs idle: each workgroup takes kc_per
+    // of the ceil(k / 256) chains, so that about 512 workgroups run in all. A 64 tile alone on its
+    // CU takes 6.3 us per chain, and the slices, their fold and the scratch cost 10-15 us, so at
+    // least three chains have to be saved. Measured (us, split / not): 512 x 2048 x 512 (64 tiles)
+    // 23.8 / 50.7, 128 x 2000 x 300 (10) 19.8 / 50.2, 64 x 1024 x 2048 (32) 20.4 / 27.1; 247 x 525 x
+    // 914 (60, three chains) 20.2 / 16.9, 512 x 512 x 2048 (256) 24.1 / 16.1.
     const int64_t nkc = (k + kKC - 1) / kKC;
     int64_t splits = 1;
     // (the slices take 4 bytes per output and 256-k block; past 1 GiB the tiles run unsplit)
-    if (tiles < 1024 && nkc > 1 && nkc * p.outputs <= (int64_t(1) << 28)) {
-        const int64_t want = (1024 + tiles - 1) / tiles;
+    if (tiles < 256 && nkc > 1 && nkc * p.outputs <= (int64_t(1) << 28)) {
+        const int64_t want = (512 + tiles - 1) / tiles;
         const int64_t per = (nkc + std::min(want, nkc) - 1) / std::min(want, nkc);
-        p.kc_per = int32_t(per);
-        splits = (nkc + per - 1) / per;
+        if (nkc - per >= 3) {
+            p.kc_per = int32_t(per);
+            splits = (nkc + per - 1) / per;
+        }
     }
     p.blocks = tiles * splits;
     if (p.blocks > int64_t(0x7fffffff)) return fail(NT_E_ARG, "matmul: too many output tiles");
-    const bool ak = k == 1 || p.a_cs == 1;
-    const bool bn = n == 1 || p.b_cs == 1;
-    {
-        // 16-byte panel loads: a view contiguous along its read axis whose other stride, batch
-        // offsets and base are 16-byte aligned
-        auto aligned = [&](const int64_t *bs, int64_t off, int64_t other, const float *base) {
-            if (off % 4 != 0 || other % 4 != 0 || (reinterpret_cast<uintptr_t>(base) & 15) != 0) return false;
-            for (int d = 0; d < r - 2; d++)
-                if (bs[d] % 4 != 0) return false;
-            return true;
-        };
-        p.avec = ak ? (p.a_cs == 1 && aligned(p.a_bs, p.a_off, p.a_rs, a))
-                    : (p.a_rs == 1 && aligned(p.a_bs, p.a_off, p.a_cs, a));
-        p.bvec = bn ? (p.b_cs == 1 && aligned(p.b_bs, p.b_off, p.b_rs, b))
-                    : (p.b_rs == 1 && aligned(p.b_bs, p.b_off, p.b_cs, b));
-    }
+    const bool ak = p.a_cs == 1;
+    const bool bn = p.b_cs == 1 || p.b_rs != 1;
     std::unique_lock<std::mutex> lk;
     if (int rc = enter(&lk)) return rc;
     hipStream_t st = ctx().stream;
-    if (splits == 1) return H == 2 ? launch_matmul<2, false>(p, ak, bn, st) : launch_matmul<1, false>(p, ak, bn, st);
+    if (splits == 1) return launch_tile<false>(T, p, ak, bn, st);
     void *sl = nullptr;
     if (int rc = scratch_alloc(size_t(nkc) * size_t(p.outputs) * sizeof(float), &sl)) return rc;
     p.slices = static_cast<float *>(sl);
-    int rc = H == 2 ? launch_matmul<2, true>(p, ak, bn, st) : launch_matmul<1, true>(p, ak, bn, st);
+    int rc = launch_tile<true>(T, p, ak, bn, st);
     if (!rc) {
         const int64_t fb = std::min<int64_t>((p.outputs + kMmThreads - 1) / kMmThreads, 4096);
         hipLaunchKernelGGL(k_fold, dim3(unsigned(fb)), dim3(kMmThreads), 0, st, p.slices, p.outputs, int(nkc), out);

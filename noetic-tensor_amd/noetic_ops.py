@@ -8,8 +8,8 @@ meaning (a `Layout` is a view read in place; outputs are fresh, contiguous and r
 `Layout` keeps src/tensor/layout.rs's view operations. There is no CPU fallback: without the built
 library every call raises `HipUnavailable`, as in `noetic_rl`.
 
-`matmul` is the reference's f32 product bit for bit (a VALU kernel: the reference's order of fma
-chains rules out the matrix cores), `matmul_half` its reduced-precision product on the matrix cores
+`matmul` is the reference's f32 product bit for bit (f32 MFMA instructions, whose products are added in
+the reference's order), `matmul_half` its reduced-precision product on the matrix cores
 (bf16 operands, f32 accumulation), and `sort_desc` CpuRef's stable descending order on the device
 for every lane length.
 """
