@@ -25,6 +25,8 @@
 // for the policy and (max, sum exp) for the reference, rescaled when its max grows (online
 // log-sum-exp); waves and then the workgroup merge them in a fixed order; per-row scalars are
 // finished in f64.
+#include <algorithm>
+
 #include "nt_launch.hpp"
 #include "nt_rows.hpp"
 #include "rl_score_kernels.hpp"
@@ -266,13 +268,56 @@ __global__ void k_kl_estimate_grad(const float *lp, const float *lr, const float
 
 // ------------------------------------------------------------------ dispatch helpers
 
+// The states of a launch with several workgroups per row. Every such launch is on the library's one
+// stream (a launch under capture takes one workgroup per row: its graph may be replayed on another).
+constexpr int kScorePartStates = 1024;
+__device__ RowState g_score_part[kScorePartStates];
+
+// This device's address of g_score_part (the host-side name is only a stand-in).
+int score_parts(RowState **out) {
+    static RowState *at = nullptr;  // (one device per process; the context's lock is held)
+    if (!at) {
+        void *ptr = nullptr;
+        if (int rc = hip_check(hipGetSymbolAddress(&ptr, HIP_SYMBOL(g_score_part)), "hipGetSymbolAddress")) return rc;
+        at = static_cast<RowState *>(ptr);
+    }
+    *out = at;
+    return 0;
+}
+
+// Workgroups per row of the scorer: one CU reads a row at about 10 GB/s per KiB in flight, so few rows
+// leave the chip idle. About 1024 workgroups, each of at least 8 chunks (two per wave in flight
+// at once), or 24 past 64 rows, where the finishing launch (2.5 us) weighs more. Measured (us, one
+// workgroup per row / this rule): 1 row of 128256 bf16 23.7 / 7.3, 16 of 151936 with a reference
+// 42.3 / 12.0, 64 of 128256 under a shared f32 mask 32.6 / 12.6, 120 of 50304 f32 18.6 / 12.6, 256 of
+// 128256 with a u8 mask 30.5 / 23.1; two workgroups per row of 400 x 32000 lost, 13.0 / 16.1.
+int score_segs(int64_t rows, int nc) {
+    if (rows > 256) return 1;
+    const int64_t g = std::min<int64_t>(kScorePartStates / rows, nc / (rows <= 64 ? 8 : 24));
+    return int(std::min<int64_t>(std::max<int64_t>(g, 1), kScoreMaxSegs));
+}
+
+// Workgroups per row of the backward (their steps are independent): about 4096, each of two steps or
+// more. Measured (us, one workgroup per row / this rule): 1 row of 128256 bf16 20.8 / 4.0, 32 of 50304
+// f32 16.6 / 5.9, 256 of 50304 bf16 19.1 / 14.5, 1024 60.9 / 56.3; 60 unaligned rows of 50001 60.7 / 14.1.
+int grad_parts(int64_t rows, int64_t vocab) {
+    const int64_t most = (vocab + 2 * kGradStep - 1) / (2 * kGradStep);
+    return int(std::max<int64_t>(1, std::min(4096 / rows, most)));
+}
+
 template <int DT, int MK, bool REF, bool KL, bool ENT>
 void pick_al_score(bool al, const ScoreP &p, int64_t rows, hipStream_t s) {
     char nm[96];
     std::snprintf(nm, sizeof nm, "nt::k_score<%d, %d, %s, %s, %s, %s>", DT, MK, rtc_bool(REF), rtc_bool(KL),
                   rtc_bool(ENT), rtc_bool(al));
-    if (al) launch_path(k_score<DT, MK, REF, KL, ENT, true>, nm, dim3(unsigned(rows)), dim3(kScoreThreads), 0, s, p);
-    else launch_path(k_score<DT, MK, REF, KL, ENT, false>, nm, dim3(unsigned(rows)), dim3(kScoreThreads), 0, s, p);
+    const dim3 grid(unsigned(rows * p.segs));
+    if (al) launch_path(k_score<DT, MK, REF, KL, ENT, true>, nm, grid, dim3(kScoreThreads), 0, s, p);
+    else launch_path(k_score<DT, MK, REF, KL, ENT, false>, nm, grid, dim3(kScoreThreads), 0, s, p);
+    if (p.segs > 1) {
+        std::snprintf(nm, sizeof nm, "nt::k_score_finish<%d, %d, %s, %s, %s>", DT, MK, rtc_bool(REF), rtc_bool(KL),
+                      rtc_bool(ENT));
+        launch_path(k_score_finish<DT, MK, REF, KL, ENT>, nm, dim3(unsigned(rows)), dim3(kWave), 0, s, p);
+    }
 }
 
 template <int DT, int MK>
@@ -348,6 +393,14 @@ int nt_hip_rl_score(const NtRlScoreArgs *a) {
               a->vocab * 4 <= int64_t(0x7fffffff);
     if (ref) al = al && reinterpret_cast<uintptr_t>(a->ref_logits) % 16 == 0;
     hipStream_t s = ctx().stream;
+    p.segs = score_segs(a->rows, p.nc);
+    p.part = nullptr;
+    if (p.segs > 1) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (int rc = hip_check(hipStreamIsCapturing(s, &cap), "hipStreamIsCapturing")) return rc;
+        if (cap != hipStreamCaptureStatusNone) p.segs = 1;
+        else if (int rc = score_parts(&p.part)) return rc;
+    }
     rtc_status() = 0;
     if (a->dtype == NT_F32) pick_mk_score<NT_F32>(a->mask_kind, ref, kl, ent, al, p, a->rows, s);
     else if (a->dtype == NT_BF16) pick_mk_score<NT_BF16>(a->mask_kind, ref, kl, ent, al, p, a->rows, s);
@@ -398,6 +451,7 @@ int nt_hip_rl_score_backward(const NtRlScoreGradArgs *a) {
     p.gkl = a->g_kl;
     p.gh = a->g_entropy;
     p.grad = a->grad;
+    p.parts = grad_parts(a->rows, a->vocab);
     const bool kl = a->g_kl != nullptr;
     // the buffer-resource path addresses a row's bytes with 32-bit offsets
     bool al = aligned_rows(a->logits, a->vocab, a->ld, a->dtype, a->mask_kind, a->mask, mm) &&
@@ -413,7 +467,8 @@ int nt_hip_rl_score_backward(const NtRlScoreGradArgs *a) {
             char nm[96];
             std::snprintf(nm, sizeof nm, "nt::k_score_grad<%d, %d, %s, %d, %s>", DT, MK, rtc_bool(KL), GDT,
                           rtc_bool(AL));
-            launch_path(k_score_grad<DT, MK, KL, GDT, AL>, nm, dim3(unsigned(a->rows)), dim3(kGradThreads), 0, s, p);
+            launch_path(k_score_grad<DT, MK, KL, GDT, AL>, nm, dim3(unsigned(a->rows * p.parts)),
+                        dim3(kGradThreads), 0, s, p);
         };
         auto by_al = [&](auto klc, auto gdt) {
             if (al) launch(klc, gdt, std::true_type{});

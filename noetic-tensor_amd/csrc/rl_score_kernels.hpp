@@ -28,6 +28,8 @@ struct ScoreP {
     float *logp, *ref_logp, *kl, *ent;
     uint8_t *status;
     float *lse_base, *lse_rest, *ref_lse_base, *ref_lse_rest;
+    int segs;               // workgroups per row
+    struct RowState *part;  // segs > 1: their states, [rows][segs]
 };
 
 // Running state of one lane (value space, exponent scale c). Every sum is relative to the
@@ -138,13 +140,78 @@ __device__ __forceinline__ void load_raw_buf(Raw<DT, MK> &r, __amdgpu_buffer_rsr
 }
 
 
+// A row's outputs from its merged state: the references af and arf, the sums relative to them in
+// f64. One thread.
+template <int DT, int MK, bool REF, bool KL, bool ENT>
+__device__ __forceinline__ void score_finish(const ScoreP &p, int64_t row, float af, float arf, double S, double H,
+                                             double B, double Sr) {
+    const bool tau_one = p.tau_one != 0;
+    const void *xrow = static_cast<const char *>(p.logits) + row * p.ld * Elem<DT>::kBytes;
+    const void *yrow = nullptr;
+    if constexpr (REF) yrow = static_cast<const char *>(p.ref) + row * p.ld * Elem<DT>::kBytes;
+    const void *mrow = nullptr;
+    if constexpr (MK != NT_MASK_NONE) mrow = static_cast<const char *>(p.mask) + mask_row_at(p.mm, row) * MaskWords<MK>::kBytes;
+    // The value-space max as the reference's f32 max of the tempered logits.
+    auto zmax = [&](float a) -> float {
+        if constexpr (MK != NT_MASK_F32) return tau_one ? a : a / p.tau;
+        else return a;
+    };
+    int stt = NT_ROW_OK;
+    // (nothing allowed, or every allowed logit below -FLT_MAX T, whose tempered value is -inf)
+    if (af == -INFINITY || zmax(af) == -INFINITY) stt = NT_ROW_NO_TOKEN;
+    else if (!(S == S)) stt = NT_ROW_NAN;
+    const double lnS = log(S);
+    // The tempered logit of one token, with the reference's f32 arithmetic.
+    auto ztok = [&](const void *rowp, int64_t tok) -> float {
+        float x;
+        if constexpr (DT == NT_F32) x = static_cast<const float *>(rowp)[tok];
+        else x = widen16<DT>(uint32_t(static_cast<const uint16_t *>(rowp)[tok]));
+        float z = tau_one ? x : x / p.tau;
+        if constexpr (MK == NT_MASK_U8) {
+            if (static_cast<const uint8_t *>(mrow)[tok] == 0) z = -INFINITY;
+        } else if constexpr (MK == NT_MASK_F32) {
+            z = z + static_cast<const float *>(mrow)[tok];
+        }
+        return z;
+    };
+    int64_t tok = -1;
+    if (p.tokens) {
+        tok = p.tokens[row];
+        if ((tok < 0 || tok >= p.V) && stt == NT_ROW_OK) stt = kRowBadToken;
+    }
+    const bool rowok = stt == NT_ROW_OK || stt == kRowBadToken;
+    if (p.logp) p.logp[row] = stt == NT_ROW_OK ? float((double(ztok(xrow, tok)) - double(zmax(af))) - lnS) : NAN;
+    if (p.ent) p.ent[row] = rowok ? float(lnS - kLn2 * H / S) : NAN;
+    // The log-sum-exp as base + rest (z units): the base is the tempered value of the row's
+    // final reference, the rest ln of the sum relative to it.
+    if (p.lse_base) p.lse_base[row] = rowok ? zmax(af) : NAN;
+    if (p.lse_rest) p.lse_rest[row] = rowok ? float(lnS) : NAN;
+    if constexpr (REF) {
+        const bool rok = arf != -INFINITY && Sr == Sr;
+        if (p.ref_lse_base) p.ref_lse_base[row] = rok ? zmax(arf) : NAN;
+        if (p.ref_lse_rest) p.ref_lse_rest[row] = rok ? float(log(Sr)) : NAN;
+        if (p.ref_logp)
+            p.ref_logp[row] = (rok && tok >= 0 && tok < p.V) ? float((double(ztok(yrow, tok)) - double(zmax(arf))) - log(Sr)) : NAN;
+        if constexpr (KL) {
+            // KL = sum p ((z - m) - (z_ref - m_ref)) - ln S + ln S_ref; the first sum is
+            // ln2 * B / S because c ln2 is the value-to-logit scale (1/T, or 1 with an f32 mask).
+            if (p.kl) p.kl[row] = (rowok && rok) ? float(kLn2 * B / S - log(S / Sr)) : NAN;
+        }
+    }
+    if (p.status) p.status[row] = uint8_t(stt);
+}
+
+// One workgroup per row, or p.segs of them: workgroup g of a row is then its waves g nw .. of segs nw,
+// and leaves its state for k_score_finish.
 template <int DT, int MK, bool REF, bool KL, bool ENT, bool AL>
 __global__ __launch_bounds__(kScoreThreads) void k_score(ScoreP p) {
     __shared__ RowState ws[kScoreWaves];
-    const int64_t row = blockIdx.x;
+    const int64_t row = blockIdx.x / unsigned(p.segs);
+    const int seg = int(blockIdx.x % unsigned(p.segs));
     const int lane = threadIdx.x & (kWave - 1);
-    const int wave = threadIdx.x / kWave;
-    const int nw = blockDim.x / kWave;
+    const int wave0 = threadIdx.x / kWave;  // in the workgroup; `wave` of `nw` in the row
+    const int wave = seg * kScoreWaves + wave0;
+    const int nw = p.segs * kScoreWaves;
     const bool tau_one = p.tau_one != 0;
     const float c = p.c;
     const void *xrow = static_cast<const char *>(p.logits) + row * p.ld * Elem<DT>::kBytes;
@@ -285,18 +352,24 @@ __global__ __launch_bounds__(kScoreThreads) void k_score(ScoreP p) {
         const RowState t = shfl_down_state(st, o);
         if (lane < o) state_merge<REF, KL, ENT>(st, t, c);
     }
-    if (lane == 0) ws[wave] = st;
+    if (lane == 0) ws[wave0] = st;
     __syncthreads();
     if (threadIdx.x != 0) return;
+    if (p.segs > 1) {
+        st = ws[0];
+        for (int i = 1; i < kScoreWaves; i++) state_merge<REF, KL, ENT>(st, ws[i], c);
+        p.part[blockIdx.x] = st;
+        return;
+    }
 
     // Finish the row in f64.
     float af = -INFINITY, arf = -INFINITY;
-    for (int i = 0; i < nw; i++) {
+    for (int i = 0; i < kScoreWaves; i++) {
         af = fmaxf(af, ws[i].a);
         arf = fmaxf(arf, ws[i].ar);
     }
     double S = 0.0, H = 0.0, B = 0.0, Sr = 0.0;
-    for (int i = 0; i < nw; i++) {
+    for (int i = 0; i < kScoreWaves; i++) {
         if (ws[i].S > 0.0f) {
             const double d = double(ws[i].a - af) * double(c);
             const double f = exp2(d);
@@ -311,54 +384,38 @@ __global__ __launch_bounds__(kScoreThreads) void k_score(ScoreP p) {
         }
         if (REF && ws[i].ar != -INFINITY) Sr += exp2(double(ws[i].ar - arf) * double(c)) * double(ws[i].Sr);
     }
-    // The value-space max as the reference's f32 max of the tempered logits.
-    auto zmax = [&](float a) -> float {
-        if constexpr (MK != NT_MASK_F32) return tau_one ? a : a / p.tau;
-        else return a;
-    };
-    int stt = NT_ROW_OK;
-    // (nothing allowed, or every allowed logit below -FLT_MAX T, whose tempered value is -inf)
-    if (af == -INFINITY || zmax(af) == -INFINITY) stt = NT_ROW_NO_TOKEN;
-    else if (!(S == S)) stt = NT_ROW_NAN;
-    const double lnS = log(S);
-    // The tempered logit of one token, with the reference's f32 arithmetic.
-    auto ztok = [&](const void *rowp, int64_t tok) -> float {
-        float x;
-        if constexpr (DT == NT_F32) x = static_cast<const float *>(rowp)[tok];
-        else x = widen16<DT>(uint32_t(static_cast<const uint16_t *>(rowp)[tok]));
-        float z = tau_one ? x : x / p.tau;
-        if constexpr (MK == NT_MASK_U8) {
-            if (static_cast<const uint8_t *>(mrow)[tok] == 0) z = -INFINITY;
-        } else if constexpr (MK == NT_MASK_F32) {
-            z = z + static_cast<const float *>(mrow)[tok];
+    score_finish<DT, MK, REF, KL, ENT>(p, row, af, arf, S, H, B, Sr);
+}
+
+// The rows of a launch with several workgroups per row: a wave per row takes each of its (at most 64)
+// states in one lane, and their sums in index order in f64.
+constexpr int kScoreMaxSegs = kWave;
+
+template <int DT, int MK, bool REF, bool KL, bool ENT>
+__global__ __launch_bounds__(kWave) void k_score_finish(ScoreP p) {
+    const int64_t row = blockIdx.x;
+    const int lane = threadIdx.x;
+    RowState s{-INFINITY, 0.0f, 0.0f, 0.0f, -INFINITY, 0.0f};
+    if (lane < p.segs) s = p.part[row * p.segs + lane];
+    const float af = wave_max(s.a), arf = REF ? wave_max(s.ar) : -INFINITY;
+    double S = 0.0, H = 0.0, B = 0.0, Sr = 0.0;
+    if (s.S > 0.0f) {
+        const double d = double(s.a - af) * double(p.c), f = exp2(d);
+        S = f * double(s.S);
+        if (ENT) H = f * (double(s.H) + d * double(s.S));
+        if (KL) {
+            const double e = s.ar == -INFINITY ? -INFINITY : double(s.ar - arf) * double(p.c);
+            B = f * (double(s.B) + (d - e) * double(s.S));
         }
-        return z;
-    };
-    int64_t tok = -1;
-    if (p.tokens) {
-        tok = p.tokens[row];
-        if ((tok < 0 || tok >= p.V) && stt == NT_ROW_OK) stt = kRowBadToken;
+    } else if (!(s.S == s.S)) {
+        S = NAN;
     }
-    const bool rowok = stt == NT_ROW_OK || stt == kRowBadToken;
-    if (p.logp) p.logp[row] = stt == NT_ROW_OK ? float((double(ztok(xrow, tok)) - double(zmax(af))) - lnS) : NAN;
-    if (p.ent) p.ent[row] = rowok ? float(lnS - kLn2 * H / S) : NAN;
-    // The log-sum-exp as base + rest (z units): the base is the tempered value of the row's
-    // final reference, the rest ln of the sum relative to it.
-    if (p.lse_base) p.lse_base[row] = rowok ? zmax(af) : NAN;
-    if (p.lse_rest) p.lse_rest[row] = rowok ? float(lnS) : NAN;
-    if constexpr (REF) {
-        const bool rok = arf != -INFINITY && Sr == Sr;
-        if (p.ref_lse_base) p.ref_lse_base[row] = rok ? zmax(arf) : NAN;
-        if (p.ref_lse_rest) p.ref_lse_rest[row] = rok ? float(log(Sr)) : NAN;
-        if (p.ref_logp)
-            p.ref_logp[row] = (rok && tok >= 0 && tok < p.V) ? float((double(ztok(yrow, tok)) - double(zmax(arf))) - log(Sr)) : NAN;
-        if constexpr (KL) {
-            // KL = sum p ((z - m) - (z_ref - m_ref)) - ln S + ln S_ref; the first sum is
-            // ln2 * B / S because c ln2 is the value-to-logit scale (1/T, or 1 with an f32 mask).
-            if (p.kl) p.kl[row] = (rowok && rok) ? float(kLn2 * B / S - log(S / Sr)) : NAN;
-        }
-    }
-    if (p.status) p.status[row] = uint8_t(stt);
+    if (REF && s.ar != -INFINITY) Sr = exp2(double(s.ar - arf) * double(p.c)) * double(s.Sr);
+    S = readlane_d(wave_scan_dpp(S), kWave - 1);
+    if (ENT) H = readlane_d(wave_scan_dpp(H), kWave - 1);
+    if (KL) B = readlane_d(wave_scan_dpp(B), kWave - 1);
+    if (REF) Sr = readlane_d(wave_scan_dpp(Sr), kWave - 1);
+    if (lane == 0) score_finish<DT, MK, REF, KL, ENT>(p, row, af, arf, S, H, B, Sr);
 }
 
 // ------------------------------------------------------------------ fused backward
@@ -382,6 +439,7 @@ struct GradP {
     const int32_t *tokens;
     const float *lb, *lr, *rlb, *rlr, *kl, *ent, *glp, *gkl, *gh;
     void *grad;
+    int parts;  // workgroups per row: each takes every parts-th step
 };
 
 constexpr int kGradThreads = 256;
@@ -517,7 +575,7 @@ __device__ __forceinline__ void grad_step(const GradRow &g, float tau, const Raw
 // a lane's elements lies wholly inside the row or wholly past it (V % 8 == 0). Every input is
 // read once and the gradient written once, so all of them are accessed non-temporally.
 template <int DT, int MK, bool KL, int GDT, bool TAU1>
-__device__ __forceinline__ void grad_row_aligned(const GradP &p, const GradRow &g, int64_t row) {
+__device__ __forceinline__ void grad_row_aligned(const GradP &p, const GradRow &g, int64_t row, int part) {
     constexpr int XB = Elem<DT>::kBytes, MB = MaskWords<MK>::kBytes, GB = GDT == NT_F32 ? 4 : 2;
     constexpr bool SPLIT = GDT == NT_F32;
     constexpr int kHalf = kGradStep / 2;
@@ -610,7 +668,8 @@ __device__ __forceinline__ void grad_row_aligned(const GradP &p, const GradRow &
     };
     const int t = int(threadIdx.x);
     const int first = SPLIT ? 4 * t : kEpl * t;  // the lane's first element in step 0
-    for (int s0 = 0; s0 < V; s0 += 2 * kGradStep) {
+    // (no overflow: V is below 2^29 and parts at most V / (2 kGradStep), rounded up)
+    for (int s0 = 2 * kGradStep * part; s0 < V; s0 += 2 * kGradStep * p.parts) {
         Raw<DT, MK> x0, x1;
         Raw<DT, NT_MASK_NONE> y0, y1;
         const int a0 = s0 + first, a1 = a0 + kGradStep;
@@ -626,13 +685,13 @@ __device__ __forceinline__ void grad_row_aligned(const GradP &p, const GradRow &
 
 // Any other row layout: element-wise bounds and plain stores.
 template <int DT, int MK, bool KL, int GDT, bool TAU1>
-__device__ __forceinline__ void grad_row_general(const GradP &p, const GradRow &g, int64_t row) {
+__device__ __forceinline__ void grad_row_general(const GradP &p, const GradRow &g, int64_t row, int part) {
     const char *xrow = static_cast<const char *>(p.logits) + row * p.ld * Elem<DT>::kBytes;
     const char *yrow = KL ? static_cast<const char *>(p.ref) + row * p.ld * Elem<DT>::kBytes : nullptr;
     const char *mrow = MK != NT_MASK_NONE ? static_cast<const char *>(p.mask) + mask_row_at(p.mm, row) * MaskWords<MK>::kBytes
                                           : nullptr;
     char *grow = static_cast<char *>(p.grad) + row * p.gld * (GDT == NT_F32 ? 4 : 2);
-    for (int64_t e0 = int64_t(threadIdx.x) * kEpl; e0 < p.V; e0 += kGradStep) {
+    for (int64_t e0 = int64_t(part) * kGradStep + threadIdx.x * kEpl; e0 < p.V; e0 += int64_t(p.parts) * kGradStep) {
         Raw<DT, MK> rx;
         Raw<DT, NT_MASK_NONE> ry;
         load_raw<DT, MK, false>(rx, xrow, mrow, e0, p.V);
@@ -654,14 +713,15 @@ __device__ __forceinline__ void grad_row_general(const GradP &p, const GradRow &
 
 template <int DT, int MK, bool KL, int GDT, bool AL>
 __global__ __launch_bounds__(kGradThreads) void k_score_grad(GradP p) {
-    const int64_t row = blockIdx.x;
+    const int64_t row = blockIdx.x / unsigned(p.parts);
+    const int part = int(blockIdx.x % unsigned(p.parts));
     const GradRow g = grad_row<KL>(p, row);
     if (p.tau_one) {
-        if constexpr (AL) grad_row_aligned<DT, MK, KL, GDT, true>(p, g, row);
-        else grad_row_general<DT, MK, KL, GDT, true>(p, g, row);
+        if constexpr (AL) grad_row_aligned<DT, MK, KL, GDT, true>(p, g, row, part);
+        else grad_row_general<DT, MK, KL, GDT, true>(p, g, row, part);
     } else {
-        if constexpr (AL) grad_row_aligned<DT, MK, KL, GDT, false>(p, g, row);
-        else grad_row_general<DT, MK, KL, GDT, false>(p, g, row);
+        if constexpr (AL) grad_row_aligned<DT, MK, KL, GDT, false>(p, g, row, part);
+        else grad_row_general<DT, MK, KL, GDT, false>(p, g, row, part);
     }
 }
 
