@@ -8,8 +8,8 @@
 //
 // Each element becomes one 64-bit key, (order key << 32) | ~position, so that a plain descending
 // comparison of keys is CpuRef's order with ties broken by position, and no two keys are equal.
-// A lane of up to kSortCap elements is sorted by one workgroup (bitonic, the keys in registers,
-// LDS only for exchanges between waves). A longer lane is
+// A lane of up to kSortCap elements is sorted by one workgroup (four counting passes over the order
+// key in LDS). A longer lane is
 // cut into kSortCap-long runs, each sorted that way into a scratch buffer, and the runs are
 // merged pairwise (merge path: each workgroup stages the two input windows that feed its tile of
 // outputs into LDS and merges them there) until one run remains. The last step writes each position's value, decoded from its key (a NaN is read back
@@ -27,22 +27,18 @@
 namespace nt {
 namespace {
 
-constexpr int kSortThreads = 1024;
-constexpr int kSortCap = 8192;   // elements one workgroup sorts in LDS (64 KB of keys)
+constexpr int kSortCap = 16384;  // elements one workgroup sorts in LDS (the longest run)
 constexpr int kMergeThreads = 256;
 constexpr int kMergeItems = 8;   // outputs per thread of a merge pass
 constexpr int kMergeTile = kMergeThreads * kMergeItems;  // outputs per workgroup (divides 2 kSortCap)
 constexpr int kWaveSize = 64;
 
-__device__ __forceinline__ uint64_t sort_key(float v, uint32_t pos) {
-    uint32_t k;
-    if (v != v) {
-        k = 0xffffffffu;  // every NaN, whatever its sign and payload, above +inf
-    } else {
-        const uint32_t b = __float_as_uint(v);
-        k = (b & 0x80000000u) ? ~b : (b | 0x80000000u);  // total_cmp's order as an unsigned key
-    }
-    return (uint64_t(k) << 32) | uint64_t(~pos);
+// CpuRef's order as an unsigned key: every NaN, whatever its sign and payload, above +inf, then
+// total_cmp's order.
+__device__ __forceinline__ uint32_t order_key(float v) {
+    if (v != v) return 0xffffffffu;
+    const uint32_t b = __float_as_uint(v);
+    return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
 
 __device__ __forceinline__ uint32_t key_pos(uint64_t c) { return ~uint32_t(c); }
@@ -62,93 +58,127 @@ struct SortP {
     uint64_t *runs;   // [lanes][n] sorted runs (multi-run lanes)
     int64_t outer, n, inner;
     int32_t chunks;   // runs per lane
-    int32_t pw;       // power of two >= the longest run (<= kSortCap)
 };
 
-// Sort run `chunk` of lane `lane`; a lane of one run is written out directly. Thread tid holds
-// positions tid + 1024 q (q < 8) in registers through the whole bitonic network, so a stage's
-// partner t ^ j is in the same thread when j >= 1024 (a register swap), in the same wave when
-// j < 64 (a lane shuffle), and only for 64 <= j < 1024 in another wave (an exchange through LDS
-// between two barriers): 22 of the 91 stages of 8192 keys touch LDS.
-__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int j) {
-    const uint32_t lo = uint32_t(v), hi = uint32_t(v >> 32);
-    return (uint64_t(uint32_t(__shfl_xor(int(hi), j))) << 32) | uint32_t(__shfl_xor(int(lo), j));
-}
-
-// The value position t keeps at stage (k, j) given its partner's: the lower position of a pair
-// takes the larger key in a descending block ((t & k) == 0), the smaller in an ascending one.
-__device__ __forceinline__ uint64_t cmp_keep(uint64_t mine, uint64_t other, int t, int j, int k) {
-    const bool lower = (t & j) == 0;
-    const bool desc = (t & k) == 0;
-    const bool take_max = lower == desc;
-    const bool mine_bigger = mine > other;
-    return (take_max == mine_bigger) ? mine : other;
-}
-
-__global__ __launch_bounds__(kSortThreads) void k_sort_runs(SortP p) {
-    __shared__ uint64_t s[kSortCap];
-    constexpr int Q = kSortCap / kSortThreads;  // keys per thread
-    const int64_t lane = blockIdx.x / p.chunks;
-    const int chunk = int(blockIdx.x - lane * p.chunks);
-    const int64_t o = lane / p.inner, i = lane - o * p.inner;
+// Sort run `chunk` of lane `lane` (at most THREADS x E elements) by four stable counting passes over
+// the key's bytes, lowest first; a lane of one run is written out directly. Wave w holds elements
+// 64 E w .. in E registers per lane, element 64 E w + 64 e + lane in register e, so (w, e, lane) is
+// their order. In a pass each wave counts its elements per digit in its own LDS row, E steps of 64
+// elements: the lanes of one digit find each other by a ballot per bit, an element's rank is the
+// count before its step plus the peers before its lane, and the last peer adds the step's peers to
+// the count (a wave's LDS operations run in order). The workgroup then sums the counts over digits
+// and waves, and each element moves to its place in LDS. Keys are stored inverted, so that the
+// ascending passes give the descending order and equal keys keep their positions; padding takes the
+// largest inverted key, above every real one. Bound by VALU issue (about 70 instructions per step and
+// pass): [64, 128256] in runs of 16384 takes 116 us; the bitonic network of 91 stages before it took
+// 254 us for runs of 8192.
+template <int THREADS, int E>
+__global__ __launch_bounds__(THREADS) void k_sort_runs(SortP p) {
+    constexpr int W = THREADS / kWaveSize, CAP = THREADS * E, D = 256;
+    __shared__ uint32_t skey[CAP];
+    __shared__ uint16_t spos[CAP];
+    __shared__ uint32_t cnt[W][D];  // a wave's counts; then each digit's exclusive sum over the waves
+    __shared__ uint32_t first[D];   // each digit's first place
+    __shared__ uint32_t wsum[D / kWaveSize];
+    const int64_t lane_id = blockIdx.x / p.chunks;
+    const int chunk = int(blockIdx.x - lane_id * p.chunks);
+    const int64_t o = lane_id / p.inner, i = lane_id - o * p.inner;
     const int64_t beg = int64_t(chunk) * kSortCap;
-    const int len = int(std::min<int64_t>(kSortCap, p.n - beg));
-    const int P = p.pw;
-    const int tid = threadIdx.x;
-    uint64_t v[Q];
+    const int len = int(std::min<int64_t>(CAP, p.n - beg));
+    const int tid = threadIdx.x, lane = tid % kWaveSize, w = tid / kWaveSize;
+    const int t0 = w * kWaveSize * E + lane;  // element of register 0
+    uint32_t key[E], pos[E], rank[E];
 #pragma unroll
-    for (int q = 0; q < Q; q++) {
-        const int t = tid + kSortThreads * q;
-        uint64_t c = 0;  // padding: below every real key (the smallest real order key is 0x007fffff)
-        if (t < len) c = sort_key(p.x[(o * p.n + beg + t) * p.inner + i], uint32_t(beg + t));
-        v[q] = c;
+    for (int e = 0; e < E; e++) {
+        const int t = t0 + e * kWaveSize;
+        key[e] = t < len ? ~order_key(p.x[(o * p.n + beg + t) * p.inner + i]) : 0xffffffffu;
+        pos[e] = uint32_t(t);
     }
-    // Positions at or past P only meet each other (t ^ j >= P for t >= P, j < P): zeros stay there.
-    for (int k = 2; k <= P; k <<= 1) {
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            if (j >= kSortThreads) {
-                const int jq = j / kSortThreads;
+#pragma unroll 1
+    for (int shift = 0; shift < 32; shift += 8) {
+        for (int d = lane; d < D; d += kWaveSize) cnt[w][d] = 0;
 #pragma unroll
-                for (int q = 0; q < Q; q++) {
-                    if (q & jq) continue;
-                    const int t = tid + kSortThreads * q;
-                    const uint64_t a = v[q], b = v[q | jq];
-                    v[q] = cmp_keep(a, b, t, j, k);
-                    v[q | jq] = cmp_keep(b, a, t + j, j, k);
-                }
-            } else if (j >= kWaveSize) {
+        for (int e = 0; e < E; e++) {
+            const uint32_t d = (key[e] >> shift) & 255u;
+            uint32_t lo = ~0u, hi = ~0u;  // the lanes of this lane's digit
 #pragma unroll
-                for (int q = 0; q < Q; q++) s[tid + kSortThreads * q] = v[q];
-                __syncthreads();
+            for (int b = 0; b < 8; b++) {
+                const uint32_t bit = uint32_t(int32_t(key[e] << (31 - shift - b)) >> 31);  // all ones or none
+                const uint64_t bal = __builtin_amdgcn_ballot_w64(bit != 0);
+                lo &= ~(uint32_t(bal) ^ bit);
+                hi &= ~(uint32_t(bal >> 32) ^ bit);
+            }
+            const uint32_t before = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+            const uint32_t total = uint32_t(__popc(lo) + __popc(hi));
+            asm volatile("" ::: "memory");
+            const uint32_t old = cnt[w][d];
+            asm volatile("" ::: "memory");
+            if (before + 1 == total) cnt[w][d] = old + total;
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_wave_barrier();
+            rank[e] = old + before;
+        }
+        __syncthreads();
+        uint32_t sum = 0, incl = 0;
+        if (tid < D) {
 #pragma unroll
-                for (int q = 0; q < Q; q++) {
-                    const int t = tid + kSortThreads * q;
-                    v[q] = cmp_keep(v[q], s[t ^ j], t, j, k);
-                }
-                __syncthreads();
-            } else {
+            for (int v = 0; v < W; v++) {
+                const uint32_t c = cnt[v][tid];
+                cnt[v][tid] = sum;
+                sum += c;
+            }
+            incl = sum;
 #pragma unroll
-                for (int q = 0; q < Q; q++) {
-                    const int t = tid + kSortThreads * q;
-                    v[q] = cmp_keep(v[q], shfl_xor_u64(v[q], j), t, j, k);
-                }
+            for (int s = 1; s < kWaveSize; s <<= 1) {
+                const uint32_t up = uint32_t(__shfl_up(int(incl), s, kWaveSize));
+                if (lane >= s) incl += up;
+            }
+            if (lane == kWaveSize - 1) wsum[w] = incl;
+        }
+        __syncthreads();
+        if (tid < D) {
+            uint32_t base = 0;
+            for (int v = 0; v < w; v++) base += wsum[v];
+            first[tid] = base + incl - sum;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const uint32_t d = (key[e] >> shift) & 255u;
+            const uint32_t at = first[d] + cnt[w][d] + rank[e];
+            skey[at] = key[e];
+            spos[at] = uint16_t(pos[e]);
+        }
+        __syncthreads();
+        if (shift < 24) {
+#pragma unroll
+            for (int e = 0; e < E; e++) {
+                key[e] = skey[t0 + e * kWaveSize];
+                pos[e] = spos[t0 + e * kWaveSize];
             }
         }
     }
-#pragma unroll
-    for (int q = 0; q < Q; q++) {
-        const int t = tid + kSortThreads * q;
-        if (t >= len) continue;
-        const uint64_t c = v[q];
+    for (int t = tid; t < len; t += THREADS) {
+        const uint32_t src = uint32_t(beg) + spos[t];
+        const uint64_t c = (uint64_t(~skey[t]) << 32) | uint64_t(~src);
         if (p.chunks == 1) {
-            const uint32_t src = key_pos(c);
             const int64_t at = (o * p.n + t) * p.inner + i;
             p.vals[at] = key_value(c, p.x, (o * p.n + src) * p.inner + i);
             p.idx[at] = int32_t(src);
         } else {
-            p.runs[lane * p.n + beg + t] = c;
+            p.runs[lane_id * p.n + beg + t] = c;
         }
     }
+}
+
+// Threads and elements per thread for runs of up to `longest` elements: the smallest that hold them.
+void launch_runs(const SortP &p, int64_t longest, int64_t blocks, hipStream_t s) {
+    const dim3 grid{unsigned(blocks)};
+    if (longest <= 256) hipLaunchKernelGGL((k_sort_runs<256, 1>), grid, dim3(256), 0, s, p);
+    else if (longest <= 1024) hipLaunchKernelGGL((k_sort_runs<256, 4>), grid, dim3(256), 0, s, p);
+    else if (longest <= 4096) hipLaunchKernelGGL((k_sort_runs<256, 16>), grid, dim3(256), 0, s, p);
+    else if (longest <= 8192) hipLaunchKernelGGL((k_sort_runs<1024, 8>), grid, dim3(1024), 0, s, p);
+    else hipLaunchKernelGGL((k_sort_runs<1024, 16>), grid, dim3(1024), 0, s, p);
 }
 
 // How many of the first d outputs of merging descending runs A (la keys) and B (lb keys) come
@@ -168,11 +198,13 @@ __device__ __forceinline__ int64_t co_rank(const uint64_t *A, int64_t la, const 
 // so they come from one pair of runs): two co-ranks in global memory bound the A and B windows
 // that feed them, both windows are staged into LDS with coalesced loads, each thread merges its
 // kMergeItems outputs from LDS (its own co-rank by a search in LDS), and the tile is written back
-// coalesced. If LAST, the outputs are the values and positions instead of keys.
+// coalesced (the windows and then the outputs in one 16 KB array, eight workgroups per CU, the
+// co-ranks' dependent loads being what a workgroup waits for: a pass over [64, 128256] 65 -> 35.9 us).
+// If LAST, the outputs are the values and positions instead of keys.
 template <bool LAST>
 __global__ __launch_bounds__(kMergeThreads) void k_merge(SortP p, const uint64_t *src, uint64_t *dst, int64_t w,
                                                          int64_t tiles_per_lane) {
-    __shared__ uint64_t sa[kMergeTile], sb[kMergeTile], so[kMergeTile];
+    __shared__ uint64_t sk[kMergeTile];  // the A window, then the B window; then the outputs
     __shared__ int64_t cr[2];
     const int tid = threadIdx.x;
     const int64_t lane = blockIdx.x / tiles_per_lane;
@@ -189,11 +221,16 @@ __global__ __launch_bounds__(kMergeThreads) void k_merge(SortP p, const uint64_t
     __syncthreads();
     const int64_t a0 = cr[0], b0 = d0 - cr[0];
     const int na = int(cr[1] - cr[0]), nb = int((d1 - cr[1]) - b0);
-    for (int e = tid; e < na; e += kMergeThreads) sa[e] = A[a0 + e];
-    for (int e = tid; e < nb; e += kMergeThreads) sb[e] = B[b0 + e];
-    __syncthreads();
-    const int dl = tid * kMergeItems;
     const int total = na + nb;
+#pragma unroll
+    for (int q = 0; q < kMergeItems; q++) {
+        const int e = tid + q * kMergeThreads;
+        if (e < total) sk[e] = e < na ? A[a0 + e] : B[b0 + e - na];
+    }
+    __syncthreads();
+    const uint64_t *sa = sk, *sb = sk + na;
+    const int dl = tid * kMergeItems;
+    uint64_t out[kMergeItems];
     if (dl < total) {
         int lo = std::max(0, dl - nb), hi = std::min(dl, na);
         while (lo < hi) {
@@ -202,16 +239,25 @@ __global__ __launch_bounds__(kMergeThreads) void k_merge(SortP p, const uint64_t
             else hi = mid;
         }
         int ia = lo, ib = dl - lo;
-        const int end = std::min(kMergeItems, total - dl);
-        for (int q = 0; q < end; q++) {
-            const bool from_a = ib >= nb || (ia < na && sa[ia] > sb[ib]);
-            so[dl + q] = from_a ? sa[ia++] : sb[ib++];
+        // (past a window's end a key of 0, below every real one; the last thread's outputs past
+        // `total` are not stored)
+        uint64_t ka = ia < na ? sa[ia] : 0, kb = ib < nb ? sb[ib] : 0;
+#pragma unroll
+        for (int q = 0; q < kMergeItems; q++) {
+            const bool from_a = ka > kb;
+            out[q] = from_a ? ka : kb;
+            if (from_a) ka = ++ia < na ? sa[ia] : 0;
+            else kb = ++ib < nb ? sb[ib] : 0;
         }
     }
     __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kMergeItems; q++)
+        if (dl + q < total) sk[dl + q] = out[q];
+    __syncthreads();
     const int64_t o = lane / p.inner, i = lane - o * p.inner;
     for (int e = tid; e < total; e += kMergeThreads) {
-        const uint64_t c = so[e];
+        const uint64_t c = sk[e];
         if constexpr (LAST) {
             const uint32_t s = key_pos(c);
             const int64_t at = (o * n + o0 + e) * p.inner + i;
@@ -246,14 +292,11 @@ int nt_hip_sort_desc(const float *x, int64_t outer, int64_t n, int64_t inner, fl
     const int64_t chunks = (n + kSortCap - 1) / kSortCap;
     if (lanes * chunks > int64_t(0x7fffffff)) return fail(NT_E_ARG, "sort_desc: too many lanes");
     p.chunks = int32_t(chunks);
-    int pw = 1;
-    while (pw < std::min<int64_t>(n, kSortCap)) pw <<= 1;
-    p.pw = pw;
     std::unique_lock<std::mutex> lk;
     if (int rc = enter(&lk)) return rc;
     hipStream_t st = ctx().stream;
     if (chunks == 1) {
-        hipLaunchKernelGGL(k_sort_runs, dim3(unsigned(lanes)), dim3(kSortThreads), 0, st, p);
+        launch_runs(p, n, lanes, st);
         return launched("k_sort_runs");
     }
     void *buf[2] = {nullptr, nullptr};
@@ -264,7 +307,7 @@ int nt_hip_sort_desc(const float *x, int64_t outer, int64_t n, int64_t inner, fl
         return rc;
     }
     p.runs = static_cast<uint64_t *>(buf[0]);
-    hipLaunchKernelGGL(k_sort_runs, dim3(unsigned(lanes * chunks)), dim3(kSortThreads), 0, st, p);
+    launch_runs(p, kSortCap, lanes * chunks, st);
     int rc = launched("k_sort_runs");
     const int64_t tiles = (n + kMergeTile - 1) / kMergeTile;
     const int64_t blocks = lanes * tiles;
