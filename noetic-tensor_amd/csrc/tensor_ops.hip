@@ -13,6 +13,7 @@
 #include <cmath>
 #include <cstdint>
 #include <string>
+#include <type_traits>
 
 #include "../../include/noetic_hip.h"
 #include "../../include/noetic_ops.h"
@@ -391,6 +392,87 @@ __global__ __launch_bounds__(kOpsThreads) void k_binary(int op, const float *__r
     }
 }
 
+// a op b where each operand's rows are contiguous (AM / BM 1) or one value per row (0), as a row
+// statistic or a scalar broadcast against rows is: a workgroup takes 4 x 256 x V columns of a row, so
+// no index is divided, and with V = 4 (16-byte aligned rows, C % 4 == 0) every access is 16 bytes.
+// Bound by HBM. [256, 50304] less a value per row: 26.9 -> 16.1 us (6.4 TB/s) over the element loop.
+constexpr int kRowsPer = 4;  // groups of 256 V columns per workgroup
+template <int OP, int V, int AM, int BM>
+__global__ __launch_bounds__(kOpsThreads) void k_binary_rows(const float *__restrict__ a, int64_t ars,
+                                                             const float *__restrict__ b, int64_t brs,
+                                                             float *__restrict__ y, int64_t rows, int64_t C) {
+    typedef float vec __attribute__((ext_vector_type(V)));
+    const int64_t c0 = int64_t(blockIdx.x) * (kRowsPer * kOpsThreads * V) + threadIdx.x * V;
+    for (int64_t row = blockIdx.y; row < rows; row += gridDim.y) {
+        const float *ar = a + row * ars, *br = b + row * brs;
+        const float as = AM ? 0.0f : ar[0], bs = BM ? 0.0f : br[0];
+        vec p[kRowsPer], q[kRowsPer];
+#pragma unroll
+        for (int u = 0; u < kRowsPer; u++) {
+            const int64_t c = c0 + u * (kOpsThreads * V);
+            p[u] = vec(as);
+            q[u] = vec(bs);
+            if (c < C) {
+                if (AM) p[u] = *reinterpret_cast<const vec *>(ar + c);
+                if (BM) q[u] = *reinterpret_cast<const vec *>(br + c);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kRowsPer; u++) {
+            const int64_t c = c0 + u * (kOpsThreads * V);
+            if (c >= C) continue;
+            vec r;
+#pragma unroll
+            for (int e = 0; e < V; e++) {
+                if constexpr (OP == NT_BIN_ADD) r[e] = p[u][e] + q[u][e];
+                else if constexpr (OP == NT_BIN_SUB) r[e] = p[u][e] - q[u][e];
+                else if constexpr (OP == NT_BIN_MUL) r[e] = p[u][e] * q[u][e];
+                else r[e] = div_f(p[u][e], q[u][e]);
+            }
+            *reinterpret_cast<vec *>(y + row * C + c) = r;
+        }
+    }
+}
+
+// Rank 1 or 2 views of at least 1024 columns with inner strides 0 or 1 (not both 0): launched here,
+// true. (Shorter rows leave most of a workgroup idle and keep the element loop.)
+bool launch_binary_rows(int op, const float *a, const View &av, const float *b, const View &bv, float *y, int R,
+                        hipStream_t s) {
+    const int64_t rows = R == 2 ? av.shape[0] : 1, C = av.shape[R - 1];
+    const int64_t am = av.st[R - 1], bm = bv.st[R - 1];
+    if (R > 2 || C < 1024 || am > 1 || bm > 1 || (am == 0 && bm == 0)) return false;
+    const int64_t ars = R == 2 ? av.st[0] : 0, brs = R == 2 ? bv.st[0] : 0;
+    a += av.off;
+    b += bv.off;
+    auto whole = [](const float *x, int64_t m, int64_t rs) {
+        return m == 0 || (reinterpret_cast<uintptr_t>(x) % 16 == 0 && rs % 4 == 0);
+    };
+    const bool v4 = C % 4 == 0 && whole(a, am, ars) && whole(b, bm, brs) && reinterpret_cast<uintptr_t>(y) % 16 == 0;
+    const int64_t per = int64_t(kRowsPer) * kOpsThreads * (v4 ? 4 : 1), bx = (C + per - 1) / per;
+    if (bx > 0x7fffffff) return false;
+    const dim3 grid(unsigned(bx), unsigned(rows < 32768 ? rows : 32768));
+    auto go = [&](auto opc) {
+        constexpr int OP = decltype(opc)::value;
+#define NT_ROWS(V, AM, BM) \
+    hipLaunchKernelGGL((k_binary_rows<OP, V, AM, BM>), grid, dim3(kOpsThreads), 0, s, a, ars, b, brs, y, rows, C)
+        if (v4) {
+            if (am && bm) NT_ROWS(4, 1, 1);
+            else if (am) NT_ROWS(4, 1, 0);
+            else NT_ROWS(4, 0, 1);
+        } else {
+            if (am && bm) NT_ROWS(1, 1, 1);
+            else if (am) NT_ROWS(1, 1, 0);
+            else NT_ROWS(1, 0, 1);
+        }
+#undef NT_ROWS
+    };
+    if (op == NT_BIN_ADD) go(std::integral_constant<int, NT_BIN_ADD>{});
+    else if (op == NT_BIN_SUB) go(std::integral_constant<int, NT_BIN_SUB>{});
+    else if (op == NT_BIN_MUL) go(std::integral_constant<int, NT_BIN_MUL>{});
+    else go(std::integral_constant<int, NT_BIN_DIV>{});
+    return true;
+}
+
 template <int R>
 __global__ __launch_bounds__(kOpsThreads) void k_mask_fill(const float *__restrict__ x, View xv,
                                                            const uint8_t *__restrict__ m, View mv, float value,
@@ -438,6 +520,111 @@ __global__ __launch_bounds__(kOpsThreads) void k_sum_last(const float *__restric
             y[row] = acc;
         }
     }
+}
+
+// The same fold of long rows, one row per workgroup: what bounds it is the eight dependent chains of
+// n / 8 adds, so one wave only adds, its eight lanes reading their chains' values from LDS 16 bytes
+// at a time, while four waves bring the row in, two tiles ahead. A tile is laid out by chain, the
+// chains 520 words apart: the stores (64 consecutive elements) and the eight lanes' reads each
+// touch distinct banks. [256, 50304]: 113 -> 31.6 us over the kernel above,
+// whose lanes read their chains from memory. (Reading 32 values ahead of the adds took 40.7.)
+constexpr int kSumTile = 4096, kSumChain = kSumTile / 8, kSumStride = kSumChain + 8;
+constexpr int kSumLoaders = 256, kSumPer = kSumTile / kSumLoaders;
+__global__ __launch_bounds__(kSumLoaders + kWave) void k_sum_long(const float *__restrict__ x, int64_t outer, int64_t n,
+                                                                  float *__restrict__ y) {
+    __shared__ __attribute__((aligned(16))) float s[2][8 * kSumStride];
+    const bool adds = threadIdx.x < kWave;
+    const int u = int(threadIdx.x) - kWave, g = threadIdx.x & 7;
+    const int64_t n8 = n - n % 8, tiles = (n8 + kSumTile - 1) / kSumTile;
+    for (int64_t row = blockIdx.x; row < outer; row += gridDim.x) {
+        const float *r = x + row * n;
+        float v0[kSumPer], v1[kSumPer];  // this loader's values of the next two tiles
+        auto load = [&](float(&v)[kSumPer], int64_t t) {
+#pragma unroll
+            for (int i = 0; i < kSumPer; i++) {
+                const int64_t j = t * kSumTile + u + kSumLoaders * i;
+                v[i] = j < n8 ? r[j] : 0.0f;
+            }
+        };
+        auto put = [&](const float(&v)[kSumPer], int b) {
+#pragma unroll
+            for (int i = 0; i < kSumPer; i++) s[b][(u & 7) * kSumStride + u / 8 + (kSumLoaders / 8) * i] = v[i];
+        };
+        float p = 0.0f;
+        auto add = [&](int64_t t, int b) {
+            const float *c = &s[b][g * kSumStride];
+            if ((t + 1) * kSumTile <= n8) {
+#pragma unroll 1
+                for (int q = 0; q < kSumChain; q += 32) {
+                    float4 w[8];
+#pragma unroll
+                    for (int i = 0; i < 8; i++) w[i] = *reinterpret_cast<const float4 *>(c + q + 4 * i);
+#pragma unroll
+                    for (int i = 0; i < 8; i++) {
+                        p = p + w[i].x;
+                        p = p + w[i].y;
+                        p = p + w[i].z;
+                        p = p + w[i].w;
+                    }
+                }
+            } else {
+                const int m = int(n8 - t * kSumTile) / 8;
+                for (int q = 0; q < m; q++) p = p + c[q];
+            }
+        };
+        if (!adds) {
+            load(v0, 0);
+            put(v0, 0);
+            load(v0, 1);
+            load(v1, 2);
+        }
+        __syncthreads();
+        for (int64_t t = 0; t < tiles; t += 2) {
+            if (adds) {
+                add(t, 0);
+            } else {
+                put(v0, 1);
+                load(v0, t + 3);
+            }
+            __syncthreads();
+            if (adds) {
+                if (t + 1 < tiles) add(t + 1, 1);
+            } else {
+                put(v1, 0);
+                load(v1, t + 4);
+            }
+            __syncthreads();
+        }
+        if (adds) {
+            const float p0 = __shfl(p, 0, 8), p1 = __shfl(p, 1, 8), p2 = __shfl(p, 2, 8), p3 = __shfl(p, 3, 8);
+            const float p4 = __shfl(p, 4, 8), p5 = __shfl(p, 5, 8), p6 = __shfl(p, 6, 8), p7 = __shfl(p, 7, 8);
+            if (threadIdx.x == 0) {
+                float acc = 0.0f;
+                acc = acc + (p0 + p4);
+                acc = acc + (p1 + p5);
+                acc = acc + (p2 + p6);
+                acc = acc + (p3 + p7);
+                for (int64_t j = n8; j < n; j++) acc = acc + r[j];
+                y[row] = acc;
+            }
+        }
+        __syncthreads();  // (the buffers are filled again by the next row)
+    }
+}
+
+int launch_sum_last(const float *x, int64_t outer, int64_t n, float *y, hipStream_t s) {
+    // A row per workgroup pays where rows are long and too few for their chains to fill the chip.
+    // Measured (us, k_sum_long / k_sum_last): 8 x 50304 31 / 41, 256 x 50304 31 / 115, 2048 x 50304
+    // 161 / 178, 1 x 4000000 1709 / 3990; 16384 x 4096 234 / 54, 4096 x 2048 131 / 6.5, 256 x 2048 13.5 / 5.9.
+    if ((n >= 4096 && outer <= 512) || (n >= 16384 && outer <= 2048)) {
+        hipLaunchKernelGGL(k_sum_long, dim3(unsigned(outer < kMaxBlocks ? outer : kMaxBlocks)), dim3(kSumLoaders + kWave),
+                           0, s, x, outer, n, y);
+    } else {
+        const int64_t per_block = kOpsThreads / 8, b = (outer + per_block - 1) / per_block;
+        hipLaunchKernelGGL(k_sum_last, dim3(unsigned(b < kMaxBlocks ? b : kMaxBlocks)), dim3(kOpsThreads), 0, s, x, outer,
+                           n, y);
+    }
+    return launched("sum");
 }
 
 // Along any other axis: the n slices added in order from zero (kernels.rs:163-171); one thread
@@ -490,16 +677,27 @@ __global__ __launch_bounds__(kBestThreads) void k_best_last(const float *__restr
             // 32-bit positions in the loop (the pick compares indices only on ties)
             float bv = r[0];
             int32_t bk = 0;
-            for (int32_t k = int32_t(threadIdx.x); k < int32_t(n); k += kBestThreads) {
-                const float e = r[k];
+            // k > bk always here, so the earlier index wins ties: take e only if it is a NaN over a
+            // number, or a larger number
+            auto take = [&](float e, int32_t k) {
                 const bool en = e != e, bn = bv != bv;
-                // k > bk always here, so the earlier index wins ties: take e only if it is a NaN
-                // over a number, or a larger number
                 if (!bn && (en || e > bv)) {
                     bv = e;
                     bk = k;
                 }
+            };
+            // (eight loads in flight: one at a time left the row's read bound by its latency, [256,
+            // 50304] 21.6 -> 12.1 us)
+            constexpr int kB = 8;
+            int64_t k = threadIdx.x;
+            for (; k + (kB - 1) * kBestThreads < n; k += kB * kBestThreads) {
+                float e[kB];
+#pragma unroll
+                for (int i = 0; i < kB; i++) e[i] = r[k + i * kBestThreads];
+#pragma unroll
+                for (int i = 0; i < kB; i++) take(e[i], int32_t(k + i * kBestThreads));
             }
+            for (; k < n; k += kBestThreads) take(r[k], int32_t(k));
             b = Best{bv, bk};
         } else {
             for (int64_t k = threadIdx.x; k < n; k += kBestThreads) b = pick(b, Best{r[k], k});
@@ -704,6 +902,7 @@ int nt_hip_binary(int32_t op, const float *a, const NtLayout *al, const float *b
     View v[2];
     const int R = simplify(ls, 2, v);
     hipStream_t s = ctx().stream;
+    if (launch_binary_rows(int(op), a, v[0], b, v[1], out, R, s)) return launched("binary");
     RANK_SWITCH(R, hipLaunchKernelGGL((k_binary<RR>), dim3(blocks_for(n)), dim3(kOpsThreads), 0, s, int(op), a, v[0],
                                       b, v[1], out, n));
     return launched("binary");
@@ -744,10 +943,7 @@ int nt_hip_reduce_dim(int32_t op, const float *x, int64_t outer, int64_t n, int6
     int32_t *idx = op == NT_RED_ARGMAX ? static_cast<int32_t *>(out) : nullptr;
     if (op == NT_RED_SUM) {
         if (last_axis) {
-            const int64_t per_block = kOpsThreads / 8;
-            int64_t b = (outer + per_block - 1) / per_block;
-            b = b > kMaxBlocks ? kMaxBlocks : b;
-            hipLaunchKernelGGL(k_sum_last, dim3(unsigned(b)), dim3(kOpsThreads), 0, s, x, outer, n, val);
+            return launch_sum_last(x, outer, n, val, s);
         } else {
             hipLaunchKernelGGL(k_sum_mid, dim3(blocks_for(lanes)), dim3(kOpsThreads), 0, s, x, outer, n, inner, val);
         }
@@ -771,8 +967,8 @@ int nt_hip_reduce_all(int32_t op, const float *x, int64_t n, float *out) {
     std::unique_lock<std::mutex> lk;
     if (int rc = enter(&lk)) return rc;
     hipStream_t s = ctx().stream;
-    if (op == NT_RED_SUM) hipLaunchKernelGGL(k_sum_last, dim3(1), dim3(kOpsThreads), 0, s, x, int64_t(1), n, out);
-    else hipLaunchKernelGGL(k_best_last, dim3(1), dim3(kBestThreads), 0, s, x, int64_t(1), n, out, (int32_t *)nullptr);
+    if (op == NT_RED_SUM) return launch_sum_last(x, 1, n, out, s);
+    hipLaunchKernelGGL(k_best_last, dim3(1), dim3(kBestThreads), 0, s, x, int64_t(1), n, out, (int32_t *)nullptr);
     return launched("reduce_all");
 }
 
