@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/noetic_hip.h"
@@ -47,6 +48,107 @@ int launched(const char *what) {
     return 0;
 }
 
+// Device blocks kept for reuse. A stream-ordered allocation and its free cost the host about 10 us
+// together, more than a small launch, and a scoring or loss call makes a dozen; from here a pair
+// takes 0.8 us. Blocks of up to kKeepBlock bytes come in size classes of eight per octave (at most an
+// eighth unused); a released one goes on its class's list and is handed out again to work queued
+// later on the library's one stream, the order that hipFreeAsync and hipMallocAsync would give it.
+// At most kKeepTotal bytes are kept: past it the blocks go back to the device's pool, and so do
+// all of them when the pool has no memory left. Calls made under capture take their memory from
+// the pool, as graph nodes. All of it under the context's lock.
+constexpr size_t kKeepBlock = size_t(128) << 20, kKeepTotal = size_t(512) << 20;
+constexpr int kKeepClasses = 8 * 28;
+struct KeptBlock {
+    int cls;
+    bool used;
+};
+struct Kept {
+    std::unordered_map<void *, KeptBlock> blocks;
+    std::vector<void *> lists[kKeepClasses];
+    size_t bytes = 0;  // on the lists
+};
+static Kept &kept() {
+    static Kept k;
+    return k;
+}
+
+// The size class of 1 <= bytes <= kKeepBlock and its block size: octave e (2^e <= size < 2^(e+1),
+// from 2^9), in eighths.
+static int size_class(size_t bytes, size_t *size) {
+    const size_t n = bytes < 512 ? 512 : bytes;
+    int e = 63 - __builtin_clzll((unsigned long long)n);
+    size_t step = size_t(1) << (e - 3), q = (n + step - 1) / step;  // 8 .. 16
+    if (q == 16) {
+        e++;
+        step *= 2;
+        q = 8;
+    }
+    *size = q * step;
+    return e * 8 + int(q - 8);
+}
+
+static size_t class_bytes(int cls) { return size_t(8 + cls % 8) << (cls / 8 - 3); }
+
+// Give every kept block of class `least` or above back to the device's pool.
+static int drop_kept(int least) {
+    Kept &k = kept();
+    for (int c = kKeepClasses - 1; c >= least; c--) {
+        while (!k.lists[c].empty()) {
+            void *p = k.lists[c].back();
+            if (int rc = hip_check(hipFreeAsync(p, ctx().stream), "hipFreeAsync")) return rc;
+            k.lists[c].pop_back();
+            k.blocks.erase(p);
+            k.bytes -= class_bytes(c);
+        }
+    }
+    return 0;
+}
+
+// `bytes` > 0 of device memory for work queued on the library stream from now on (pools only).
+static int take_block(size_t bytes, void **out) {
+    Ctx &c = ctx();
+    Kept &k = kept();
+    size_t size = bytes;
+    int cls = -1;
+    if (bytes <= kKeepBlock) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (int rc = hip_check(hipStreamIsCapturing(c.stream, &cap), "hipStreamIsCapturing")) return rc;
+        if (cap == hipStreamCaptureStatusNone) {
+            cls = size_class(bytes, &size);
+            if (!k.lists[cls].empty()) {
+                *out = k.lists[cls].back();
+                k.lists[cls].pop_back();
+                k.bytes -= size;
+                k.blocks[*out].used = true;
+                return 0;
+            }
+        }
+    }
+    hipError_t e = hipMallocAsync(out, size, c.stream);
+    if (e == hipErrorOutOfMemory && k.bytes > 0) {
+        (void)hipGetLastError();
+        if (int rc = drop_kept(0)) return rc;
+        e = hipMallocAsync(out, size, c.stream);
+    }
+    if (e != hipSuccess) return hip_check(e, "hipMallocAsync");
+    if (cls >= 0) k.blocks[*out] = KeptBlock{cls, true};
+    return 0;
+}
+
+static int give_block(void *p) {
+    Kept &k = kept();
+    auto it = k.blocks.find(p);
+    if (it == k.blocks.end()) return hip_check(hipFreeAsync(p, ctx().stream), "hipFreeAsync");
+    if (!it->second.used) return hip_check(hipErrorInvalidValue, "free of a block that is not in use");
+    it->second.used = false;
+    k.lists[it->second.cls].push_back(p);
+    k.bytes += class_bytes(it->second.cls);
+    // the larger blocks first: from 1 MiB (class 8 * 20) up, then all
+    if (k.bytes > kKeepTotal)
+        if (int rc = drop_kept(8 * 20)) return rc;
+    return k.bytes > kKeepTotal ? drop_kept(0) : 0;
+}
+
 // Pointers released by nt_hip_free since the last entry, freed on the stream by the next one
 // (the reference's PENDING_FREE, src/tensor/cuda/backend.rs:35-45 and 222-243: a release only
 // records the pointer, so it never waits for the device or for the context's lock).
@@ -79,7 +181,7 @@ int enter(std::unique_lock<std::mutex> *out) {
         void *p = freed[i];
         int rc = 0;
         if (c.pools) {
-            rc = hip_check(hipFreeAsync(p, c.stream), "hipFreeAsync");
+            rc = give_block(p);
         } else {
             rc = hip_check(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
             if (!rc) rc = hip_check(hipFree(p), "hipFree");
@@ -98,13 +200,13 @@ int enter(std::unique_lock<std::mutex> *out) {
 int scratch_alloc(size_t bytes, void **out) {
     *out = nullptr;
     if (bytes == 0) return 0;
-    if (ctx().pools) return hip_check(hipMallocAsync(out, bytes, ctx().stream), "hipMallocAsync");
+    if (ctx().pools) return take_block(bytes, out);
     return hip_check(hipMalloc(out, bytes), "hipMalloc");
 }
 
 int scratch_release(void *ptr) {
     if (!ptr) return 0;
-    if (ctx().pools) return hip_check(hipFreeAsync(ptr, ctx().stream), "hipFreeAsync");
+    if (ctx().pools) return give_block(ptr);
     std::lock_guard<std::mutex> pl(g_pending_mu);
     g_pending.push_back(ptr);
     return 0;
@@ -242,7 +344,7 @@ int nt_hip_alloc(size_t bytes, void **out) {
     if (bytes == 0) return 0;
     // From the device's stream-ordered pool when it has one (cuMemAllocAsync in the reference,
     // src/tensor/cuda/backend.rs:245-264): usable by work queued on the library stream after it.
-    if (ctx().pools) return hip_check(hipMallocAsync(out, bytes, ctx().stream), "hipMallocAsync");
+    if (ctx().pools) return take_block(bytes, out);
     return hip_check(hipMalloc(out, bytes), "hipMalloc");
 }
 
