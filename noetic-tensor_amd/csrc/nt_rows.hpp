@@ -101,6 +101,11 @@ struct Raw {
     uint32_t m[MaskWords<MK>::kWords > 0 ? MaskWords<MK>::kWords : 1];
 };
 
+// Words at the alignment of the f32, 16-bit or byte elements they hold.
+typedef uint32_t u32x4_f32 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x4_f16 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x2_u8 __attribute__((ext_vector_type(2), aligned(1)));
+
 // Load the 8 elements at e0 of a row. AL: the row and mask are 16-/8-byte aligned and V % 8
 // == 0, so a lane's 8 elements are all inside the row or all outside it. Elements outside
 // the row read as -inf logits.
@@ -133,6 +138,35 @@ __device__ __forceinline__ void load_raw(Raw<DT, MK> &r, const void *xrow, const
             for (int i = 0; i < Elem<DT>::kWords; i++) r.x[i] = Elem<DT>::kNegInf;
 #pragma unroll
             for (int i = 0; i < (MaskWords<MK>::kWords > 0 ? MaskWords<MK>::kWords : 1); i++) r.m[i] = 0;
+        }
+    } else if (e0 + kEpl <= V) {
+        // the lane's elements are all inside the row: the same loads at the elements' own alignment
+        // (gfx950 takes them at any byte address; the element-wise loads below are 8 to 24 a lane)
+        if constexpr (DT == NT_F32) {
+            const u32x4_f32 *q = reinterpret_cast<const u32x4_f32 *>(static_cast<const float *>(xrow) + e0);
+            const u32x4_f32 a = q[0], b = q[1];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                r.x[i] = a[i];
+                r.x[4 + i] = b[i];
+            }
+        } else {
+            const u32x4_f16 a = *reinterpret_cast<const u32x4_f16 *>(static_cast<const uint16_t *>(xrow) + e0);
+#pragma unroll
+            for (int i = 0; i < 4; i++) r.x[i] = a[i];
+        }
+        if constexpr (MK == NT_MASK_U8) {
+            const u32x2_u8 k = *reinterpret_cast<const u32x2_u8 *>(static_cast<const uint8_t *>(mrow) + e0);
+            r.m[0] = k[0];
+            r.m[1] = k[1];
+        } else if constexpr (MK == NT_MASK_F32) {
+            const u32x4_f32 *q = reinterpret_cast<const u32x4_f32 *>(static_cast<const float *>(mrow) + e0);
+            const u32x4_f32 a = q[0], b = q[1];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                r.m[i] = a[i];
+                r.m[4 + i] = b[i];
+            }
         }
     } else {
 #pragma unroll

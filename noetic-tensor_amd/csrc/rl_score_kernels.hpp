@@ -683,7 +683,8 @@ __device__ __forceinline__ void grad_row_aligned(const GradP &p, const GradRow &
     }
 }
 
-// Any other row layout: element-wise bounds and plain stores.
+// Any other row layout: loads and stores at the elements' own alignment, element-wise only where a
+// lane's 8 elements cross the row's end.
 template <int DT, int MK, bool KL, int GDT, bool TAU1>
 __device__ __forceinline__ void grad_row_general(const GradP &p, const GradRow &g, int64_t row, int part) {
     const char *xrow = static_cast<const char *>(p.logits) + row * p.ld * Elem<DT>::kBytes;
@@ -698,6 +699,17 @@ __device__ __forceinline__ void grad_row_general(const GradP &p, const GradRow &
         if constexpr (KL) load_raw<DT, NT_MASK_NONE, false>(ry, yrow, nullptr, e0, p.V);
         float o[kEpl];
         grad_step<DT, MK, KL, TAU1>(g, p.tau, rx, ry, e0, 0, o);
+        if (e0 + kEpl <= p.V) {
+            if constexpr (GDT == NT_F32) {
+                u32x4_f32 *d = reinterpret_cast<u32x4_f32 *>(reinterpret_cast<float *>(grow) + e0);
+                d[0] = u32x4_f32{__float_as_uint(o[0]), __float_as_uint(o[1]), __float_as_uint(o[2]), __float_as_uint(o[3])};
+                d[1] = u32x4_f32{__float_as_uint(o[4]), __float_as_uint(o[5]), __float_as_uint(o[6]), __float_as_uint(o[7])};
+            } else {
+                *reinterpret_cast<u32x4_f16 *>(reinterpret_cast<uint16_t *>(grow) + e0) =
+                    u32x4_f16{pack16<GDT>(o[0], o[1]), pack16<GDT>(o[2], o[3]), pack16<GDT>(o[4], o[5]), pack16<GDT>(o[6], o[7])};
+            }
+            continue;
+        }
         for (int j = 0; j < kEpl; j += 2) {
             if constexpr (GDT == NT_F32) {
                 if (e0 + j < p.V) reinterpret_cast<float *>(grow)[e0 + j] = o[j];
