@@ -7,23 +7,31 @@
 // f32, then an add kernel and an argmax kernel). Here the noise is generated where it is used:
 // ChaCha20 is a counter-mode stream, so word w of the keystream is word w % 16 of block w / 16
 // and every element's u64 is computed from the stream's key and starting word position alone.
-// One workgroup takes one row (rl_gumbel_kernels.hpp):
+// One workgroup takes one row, or a segment of one where rows are fewer than CUs (k_gumbel_finish then
+// merges the segments' records) (rl_gumbel_kernels.hpp):
 //  - the row is cut into blocks of 8 elements, one keystream block each; a block whose eight
 //    logits are all excluded (-inf) is skipped without generating it (such an element can never
 //    be the maximum of an accepted row; a row with no other candidate is refused);
 //  - each wave queues its blocks that hold an allowed element in LDS and generates their
-//    keystream by full waves;
-//  - every allowed element's draw is first screened in f32 (hardware logarithms, within 1e-5 of
-//    the exact f32 value); only the elements within a margin of the row's largest screened value
+//    keystream by full waves (a wave whose 64 blocks all do takes them from its registers);
+//  - every allowed element's value is bounded from above with two hardware logarithms of its high
+//    word; the few that come near the largest seen are screened in f32 (within 1e-5 of the exact
+//    f32 value), and only the elements within a margin of the row's largest screened value
 //    (1e-3, or four ulps of it where that is wider) can be the row's maximum. A single one is the
 //    answer; several are evaluated exactly, in f64 as the reference does, and the row's first
 //    maximum is taken among them with "greater value, else smaller index", which is associative,
 //    so the result is the sequential first maximum whatever the timing (a thread with more than
 //    four candidates sends its row to the exact evaluation of every element);
-//  - rows whose first u64 starts a block, on aligned rows, read a block's 8 logits and mask
-//    entries with vector loads issued two steps ahead; others read element by element.
+//  - a block's 8 logits and mask entries come in vector loads issued two steps ahead, at whatever
+//    alignment the stream's position and the row give them.
+// What bounds it is VALU issue: a keystream block is 936 operations a lane of about 1200 for its 8
+// draws. [256, 128256] bf16: 157 -> 134.5 us without a mask (a bound of 11 operations where every draw
+// was screened and divided), 83 -> 76.7 us under a grammar mask of runs (30% kept); sharing what the
+// waves' queues have left over the workgroup (a barrier, then 8 of 16 waves) changed nothing there
+// and cost 4 us on rows without a mask.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -41,8 +49,39 @@ template <int DT, int MK, bool ODD, bool GREEDY>
 void launch_gumbel(const GumbelP &p, int64_t rows, int threads, hipStream_t s) {
     char nm[96];
     std::snprintf(nm, sizeof nm, "nt::k_sample_gumbel<%d, %d, %s, %s>", DT, MK, rtc_bool(ODD), rtc_bool(GREEDY));
-    launch_path(k_sample_gumbel<DT, MK, ODD, GREEDY>, nm, dim3(unsigned(rows)), dim3(threads),
-                gumbel_queue_bytes(threads, GREEDY), s, p);
+    launch_path(k_sample_gumbel<DT, MK, ODD, GREEDY>, nm, dim3(unsigned(rows * p.segs)), dim3(threads),
+                gumbel_queue_bytes(threads, GREEDY, DT, MK), s, p);
+    if (p.segs > 1) {
+        std::snprintf(nm, sizeof nm, "nt::k_gumbel_finish<%d, %d, %s, %s>", DT, MK, rtc_bool(ODD), rtc_bool(GREEDY));
+        launch_path(k_gumbel_finish<DT, MK, ODD, GREEDY>, nm, dim3(unsigned(rows)), dim3(kGumbelMaxThreads),
+                    gumbel_queue_bytes(kGumbelMaxThreads, GREEDY, DT, MK), s, p);
+    }
+}
+
+// The records of a launch with several workgroups per row. Every such launch is on the library's one
+// stream (a launch under capture takes one workgroup per row: its graph may be replayed on another).
+constexpr int kGumbelRecs = 256;
+__device__ GumbelRec g_gumbel_rec[kGumbelRecs];
+
+// This device's address of g_gumbel_rec (the host-side name is only a stand-in).
+int gumbel_recs(GumbelRec **out) {
+    static GumbelRec *at = nullptr;  // (one device per process; the context's lock is held)
+    if (!at) {
+        void *ptr = nullptr;
+        if (int rc = hip_check(hipGetSymbolAddress(&ptr, HIP_SYMBOL(g_gumbel_rec)), "hipGetSymbolAddress")) return rc;
+        at = static_cast<GumbelRec *>(ptr);
+    }
+    *out = at;
+    return 0;
+}
+
+// Workgroups per row: about one per CU, each of at least 128 blocks (more pay their start, their partial
+// last step and their reductions again). Measured (us, one workgroup per row / this rule): 1 row of
+// 32000 f32 44.9 / 9.8, 16 of 50304 bf16 66.3 / 12.3, 64 of 32001 f32 48.9 / 18.6, 128 of 128256 bf16
+// under a shared f32 mask 81.7 / 51.8; with twice the workgroups 9.8, 12.5, 17.3 and 62.0.
+int gumbel_segs(int64_t rows, int64_t nblk) {
+    const int64_t g = std::min<int64_t>(256 / rows, nblk / 128);
+    return int(std::min<int64_t>(std::max<int64_t>(g, 1), 64));
 }
 
 template <int DT, int MK>
@@ -115,11 +154,22 @@ extern "C" int nt_hip_rl_sample_gumbel(const NtRlGumbelArgs *a) {
                            (mm.ld_s * msz) % (a->mask_kind == NT_MASK_F32 ? 16 : 8) == 0);
     p.vec = reinterpret_cast<uintptr_t>(a->logits) % 16 == 0 && (a->ld * esz) % 16 == 0 && mask_vec && V % 8 == 0 &&
             V * 4 <= int64_t(0x7fffffff);
-    // Threads per row: one per keystream block of the row, in whole waves, at most 1024.
-    const int64_t nblk = V / 8 + 2;
-    int threads = int(((nblk + 63) / 64) * 64);
-    threads = threads > kGumbelMaxThreads ? kGumbelMaxThreads : threads;
+    p.inv_tau = p.tau_one || a->mask_kind == NT_MASK_F32 ? 1.0f : 1.0f / p.tau;
+    p.m_ovf = p.tau_one || a->mask_kind == NT_MASK_F32 ? -INFINITY : neg_overflow_bound(p.tau);
+    p.col = chacha_columns(p.key);
     hipStream_t s = ctx().stream;
+    const int64_t nblk = V / 8 + 2;
+    p.segs = gumbel_segs(rows, nblk);
+    p.rec = nullptr;
+    if (p.segs > 1) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (int rc = hip_check(hipStreamIsCapturing(s, &cap), "hipStreamIsCapturing")) return rc;
+        if (cap != hipStreamCaptureStatusNone) p.segs = 1;
+        else if (int rc = gumbel_recs(&p.rec)) return rc;
+    }
+    // Threads per workgroup: one per keystream block of its segment, in whole waves, at most 1024.
+    int threads = int((((nblk + p.segs - 1) / p.segs + 63) / 64) * 64);
+    threads = threads > kGumbelMaxThreads ? kGumbelMaxThreads : threads;
     rtc_status() = 0;
     if (a->dtype == NT_F32) pick_gumbel_mk<NT_F32>(a->mask_kind, odd, greedy, p, rows, threads, s);
     else if (a->dtype == NT_BF16) pick_gumbel_mk<NT_BF16>(a->mask_kind, odd, greedy, p, rows, threads, s);
