@@ -77,13 +77,70 @@ struct ReadoutP {
     float *logits;       // [rows][V] debug copy or null
 };
 
+// The product of a tile for up to 64 rows: acc += over all S k-steps, each wave its 64 columns for
+// every row group. With so few rows the weight's stream from HBM is what bounds the launch (a k-step's
+// MFMAs take 64 RG cycles of a SIMD, its 8 KiB of weight about 700 at the chip's read rate), so nothing
+// is shared through LDS: each wave keeps D k-steps of its own weight fragments in flight in registers,
+// and reads h's fragments (1 KiB a row group and k-step, from the caches: every wave reads the same)
+// DH steps ahead. The same MFMA over the same k order as the pipeline of 256 rows, so the logits are
+// the same bits. Few registers and no LDS here let two workgroups share a CU. h [rows, 4096], V 128256:
+// pass 1 in 172 us at 1 row (6.1 TB/s of weight) and 189 at 64; a decode step of 1 row 248.5 -> 230, of
+// 8 rows of h [8, 1024] and V 50304 85.6 -> 70.9. Four row groups this way lost to the pipeline, 298
+// against 264 us at 128 rows, the caches' reads of h then weighing as much as the weight's.
+template <int RG>
+__device__ __forceinline__ void stream_tile(__amdgpu_buffer_rsrc_t hres, int hoff, const void *w, int woff, int S,
+                                            f32x16_t (&acc)[RG][2]) {
+    constexpr int D = 8, DH = RG == 1 ? 8 : 4;
+    static_assert(D % DH == 0, "the h ring's slots repeat within a pass of the weight's");
+    const __amdgpu_buffer_rsrc_t wres =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(w), short(0), S * 8192, kBufferWord3);
+    v4u wr[D][2], hr[DH][RG];
+    // (past the last step the loads are out of range: zeros, no memory touched)
+    auto load_w = [&](v4u(&d)[2], int t) {
+        d[0] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(wres, woff + t * 8192, 0, 0));
+        d[1] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(wres, woff + t * 8192 + 1024, 0, 0));
+    };
+    auto load_h = [&](v4u(&d)[RG], int t) {
+#pragma unroll
+        for (int g = 0; g < RG; g++)
+            d[g] = __builtin_bit_cast(
+                v4u, __builtin_amdgcn_raw_buffer_load_b128(hres, t < S ? hoff + (g * S + t) * 1024 : 0x7fffffff, 0, 0));
+    };
+#pragma unroll
+    for (int u = 0; u < D; u++) {
+        load_w(wr[u], u);
+        if (u < DH) load_h(hr[u], u);
+    }
+    for (int t0 = 0; t0 < S; t0 += D) {
+#pragma unroll
+        for (int u = 0; u < D; u++) {
+            const int t = t0 + u;
+            if (t < S) {
+#pragma unroll
+                for (int g = 0; g < RG; g++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++)
+                        acc[g][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, wr[u][j]),
+                                                                            __builtin_bit_cast(bf16x8_t, hr[u % DH][g]),
+                                                                            acc[g][j], 0, 0, 0);
+            }
+            load_w(wr[u], t + D);
+            load_h(hr[u % DH], t + DH);
+        }
+    }
+}
+
 // FIRST: the tile records carry each row's first column of the maximum (the greedy draw's
 // answer); the sampler otherwise needs only the maximum. ENT: each block also records the sum
 // of w y over its columns (w = 2^y, y = x c - tref), the entropy's term. TOKX: the lane holding
 // a row's token column writes that logit (-inf if excluded) for the scorer.
-template <bool MASK, bool DBG, bool FIRST, bool ENT, bool TOKX>
-__global__ __launch_bounds__(kRoThreads) void k_readout_tiles(ReadoutP p) {
-    __shared__ __attribute__((aligned(16))) uint8_t lds[kRoStages * kRoStageBytes];
+// RG: row groups of 32 the launch is built for, 8 (the pipeline of 256 rows, nt_mfma_pipe.hpp) or 1 or
+// 2 for up to 32 or 64 rows (stream_tile).
+template <bool MASK, bool DBG, bool FIRST, bool ENT, bool TOKX, int RG>
+__global__ __launch_bounds__(kRoThreads, RG == 8 ? 1 : 2) void k_readout_tiles(ReadoutP p) {
+    constexpr int kRows = 32 * RG;
+    constexpr int kLds = RG == 8 ? kRoStages * kRoStageBytes : kRows * kRoCols + 8 * kRows * 4;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[kLds];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // this wave's columns 64 wave .. + 63
     const int tile = blockIdx.x;
@@ -103,15 +160,16 @@ __global__ __launch_bounds__(kRoThreads) void k_readout_tiles(ReadoutP p) {
     const uint64_t wbase = reinterpret_cast<uint64_t>(p.wp + int64_t(tile) * S * 8192);
     const v4u wrs = {uint32_t(wbase), uint32_t(wbase >> 32), uint32_t(S * 8192), uint32_t(kBufferWord3)};
     // the product over the k-steps (the weight as the A operand: see the epilogue)
-    f32x16_t acc[8][2];
+    f32x16_t acc[RG][2];
 #pragma unroll
-    for (int i = 0; i < 8; i++)
+    for (int i = 0; i < RG; i++)
 #pragma unroll
         for (int j = 0; j < 2; j++)
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[i][j][v] = 0.0f;
     MfmaPipe<true> pp;
-    pp.run(lds, hres, hoff, wrs, woff, S, wave, lane, acc);
+    if constexpr (RG == 8) pp.run(lds, hres, hoff, wrs, woff, S, wave, lane, acc);
+    else stream_tile<RG>(hres, lane * 16, reinterpret_cast<const void *>(wbase), woff, S, acc);
     // ---- epilogue, in the MFMA output's own layout. The product is the transposed block, so lane
     // l of wave w holds in acc[i][j][4 a + b] row r = 32 i + l % 32 at tile column
     // 64 w + 32 j + 8 a + 4 (l / 32) + b (j < 2, a < 4, b < 4): 32 of the row's 64 columns of this
@@ -124,31 +182,31 @@ __global__ __launch_bounds__(kRoThreads) void k_readout_tiles(ReadoutP p) {
     const int el = int(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)));
     const int rw = el & 31, hh = el >> 5;
     const int cw0 = n0 + 64 * wave + 4 * hh;  // column of acc[i][0][0]; + 32 j + 8 a + b
-    // The tile's mask (256 rows x 256 bytes) comes into LDS by coalesced 1 KiB copies, four rows
+    // The tile's mask (its rows x 256 bytes) comes into LDS by coalesced 1 KiB copies, four rows
     // each, over the stages (every wave is past its last read of them after the barrier). Row r's
     // sixteen 16-byte chunks sit rotated by r (chunk k at position (k + r) % 16), so that the 32
     // lanes of a half, reading one column of 32 consecutive rows, spread over the banks. Rows past
     // the last and bytes past the mask read as zeros (the buffer's range); columns past the
     // vocabulary are excluded below. Rows that are not 16-byte aligned take byte loads instead.
     // The last odd step's MFMAs run while the copies are in flight.
-    uint8_t *const lmask = lds;                                           // [256 rows][256 bytes]
-    float *const Sm = reinterpret_cast<float *>(lds + kRoRows * kRoCols);  // [4 waves][256 rows] maxima
-    int *const Sf = reinterpret_cast<int *>(Sm + 4 * kRoRows);            // [4 waves][256 rows] first columns
-    static_assert(kRoRows * kRoCols + 8 * kRoRows * 4 <= kRoStages * kRoStageBytes, "the mask and the exchange fit");
+    uint8_t *const lmask = lds;                                           // [rows][256 bytes]
+    float *const Sm = reinterpret_cast<float *>(lds + kRows * kRoCols);  // [4 waves][rows] maxima
+    int *const Sf = reinterpret_cast<int *>(Sm + 4 * kRows);            // [4 waves][rows] first columns
+    static_assert(kRows * kRoCols + 8 * kRows * 4 <= kLds, "the mask and the exchange fit");
     const bool mdma = MASK && p.mask_vec;
     asm volatile("s_barrier" ::: "memory");
     if (mdma) {
         const __amdgpu_buffer_rsrc_t mres = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<uint8_t *>(p.mask), short(0), int((int64_t(p.rows) - 1) * p.mask_ld + p.V), kBufferWord3);
 #pragma unroll
-        for (int qq = 0; qq < kRoRows / 16; qq++) {
+        for (int qq = 0; qq < kRows / 16; qq++) {
             const int q = 4 * qq + wave;  // four rows per copy, copy q by wave q % 4
             const int r = 4 * q + (el >> 4), pos = el & 15, k = (pos - r) & 15;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(mres, (lds_ptr_t)(lmask + q * 1024), 16,
                                                      int(int64_t(r) * p.mask_ld) + n0 + 16 * k, 0, 0, 0);
         }
     }
-    pp.last_odd_step(S, acc);  // (S odd) while the copies are in flight
+    if constexpr (RG == 8) pp.last_odd_step(S, acc);  // (S odd) while the copies are in flight
 
     if (mdma) {
         wait_vmcnt<0>();
@@ -156,26 +214,26 @@ __global__ __launch_bounds__(kRoThreads) void k_readout_tiles(ReadoutP p) {
     }
     // the scored token of each of this lane's rows, relative to its first column (loaded once the
     // weight ring's registers are free; with the debug copy of the logits, one row at a time)
-    int tkd[8];
+    int tkd[RG];
     if constexpr (TOKX && !DBG) {
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
+        for (int i = 0; i < RG; i++) {
             const int r = 32 * i + rw;
             tkd[i] = p.tokens[r < p.rows ? r : 0] - cw0;
         }
     }
     // per (i, j, a) the row's four bytes at column cw0 + 32 j + 8 a (all ones without a mask);
     // zero for a row past the last, so that the byte test below also excludes it
-    uint32_t mk[8][2][4];
+    uint32_t mk[RG][2][4];
 #pragma unroll
-    for (int i = 0; i < 8; i++)
+    for (int i = 0; i < RG; i++)
 #pragma unroll
         for (int j = 0; j < 2; j++)
 #pragma unroll
             for (int a4 = 0; a4 < 4; a4++) mk[i][j][a4] = 32 * i + rw < p.rows ? 0xffffffffu : 0u;
     if constexpr (MASK) {
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
+        for (int i = 0; i < RG; i++) {
             const int r = 32 * i + rw;
             if (r >= p.rows) continue;
 #pragma unroll
@@ -202,7 +260,7 @@ __global__ __launch_bounds__(kRoThreads) void k_readout_tiles(ReadoutP p) {
         }
     }
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
+    for (int i = 0; i < RG; i++) {
         const int r = 32 * i + rw;
         const bool live = r < p.rows;
         if constexpr (DBG) {
@@ -270,13 +328,13 @@ __global__ __launch_bounds__(kRoThreads) void k_readout_tiles(ReadoutP p) {
             m = fmaxf(m, om);
         }
         if (hh == 0) {
-            Sm[wave * kRoRows + r] = m;
-            if constexpr (FIRST) Sf[wave * kRoRows + r] = first;
+            Sm[wave * kRows + r] = m;
+            if constexpr (FIRST) Sf[wave * kRows + r] = first;
         }
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every wave's maxima in LDS
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
+    for (int i = 0; i < RG; i++) {
         const int r = 32 * i + rw;
         const bool live = r < p.rows;
         // the tile's maximum and first column (the waves in column order; a tie keeps the earlier)
@@ -285,10 +343,10 @@ __global__ __launch_bounds__(kRoThreads) void k_readout_tiles(ReadoutP p) {
         if constexpr (FIRST) F = Sf[r];
 #pragma unroll
         for (int w2 = 1; w2 < 4; w2++) {
-            const float m2 = Sm[w2 * kRoRows + r];
+            const float m2 = Sm[w2 * kRows + r];
             if (m2 > M) {
                 M = m2;
-                if constexpr (FIRST) F = Sf[w2 * kRoRows + r];
+                if constexpr (FIRST) F = Sf[w2 * kRows + r];
             }
         }
         const float ref = M * p.c;  // RN(max c); -inf when nothing is allowed
@@ -1001,13 +1059,19 @@ int readout_run(const ReadoutCall &c) {
     p.logits = c.logits;
     hipStream_t st = ctx().stream;
     const dim3 g1{unsigned(ntile), 1, 1}, b1{unsigned(kRoThreads), 1, 1};
-    auto launch1 = [&](auto mask_c, auto dbg_c) {
+    auto launch_rg = [&](auto mask_c, auto dbg_c, auto rg_c) {
         constexpr bool MK = decltype(mask_c)::value, DB = decltype(dbg_c)::value;
-        if (c.greedy) hipLaunchKernelGGL((k_readout_tiles<MK, DB, true, false, false>), g1, b1, 0, st, p);
-        else if (ent && tokx) hipLaunchKernelGGL((k_readout_tiles<MK, DB, false, true, true>), g1, b1, 0, st, p);
-        else if (ent) hipLaunchKernelGGL((k_readout_tiles<MK, DB, false, true, false>), g1, b1, 0, st, p);
-        else if (tokx) hipLaunchKernelGGL((k_readout_tiles<MK, DB, false, false, true>), g1, b1, 0, st, p);
-        else hipLaunchKernelGGL((k_readout_tiles<MK, DB, false, false, false>), g1, b1, 0, st, p);
+        constexpr int RG = decltype(rg_c)::value;
+        if (c.greedy) hipLaunchKernelGGL((k_readout_tiles<MK, DB, true, false, false, RG>), g1, b1, 0, st, p);
+        else if (ent && tokx) hipLaunchKernelGGL((k_readout_tiles<MK, DB, false, true, true, RG>), g1, b1, 0, st, p);
+        else if (ent) hipLaunchKernelGGL((k_readout_tiles<MK, DB, false, true, false, RG>), g1, b1, 0, st, p);
+        else if (tokx) hipLaunchKernelGGL((k_readout_tiles<MK, DB, false, false, true, RG>), g1, b1, 0, st, p);
+        else hipLaunchKernelGGL((k_readout_tiles<MK, DB, false, false, false, RG>), g1, b1, 0, st, p);
+    };
+    auto launch1 = [&](auto mask_c, auto dbg_c) {
+        if (rows <= 32) launch_rg(mask_c, dbg_c, std::integral_constant<int, 1>{});
+        else if (rows <= 64) launch_rg(mask_c, dbg_c, std::integral_constant<int, 2>{});
+        else launch_rg(mask_c, dbg_c, std::integral_constant<int, 8>{});
     };
     if (c.logits) {
         if (p.mask) launch1(std::true_type{}, std::true_type{});
