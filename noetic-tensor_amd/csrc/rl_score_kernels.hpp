@@ -206,8 +206,12 @@ __device__ __forceinline__ void score_finish(const ScoreP &p, int64_t row, float
 template <int DT, int MK, bool REF, bool KL, bool ENT, bool AL>
 __global__ __launch_bounds__(kScoreThreads) void k_score(ScoreP p) {
     __shared__ RowState ws[kScoreWaves];
-    const int64_t row = blockIdx.x / unsigned(p.segs);
-    const int seg = int(blockIdx.x % unsigned(p.segs));
+    int64_t row = blockIdx.x;
+    int seg = 0;
+    if (p.segs > 1) {
+        row = blockIdx.x / unsigned(p.segs);
+        seg = int(blockIdx.x % unsigned(p.segs));
+    }
     const int lane = threadIdx.x & (kWave - 1);
     const int wave0 = threadIdx.x / kWave;  // in the workgroup; `wave` of `nw` in the row
     const int wave = seg * kScoreWaves + wave0;
@@ -725,8 +729,12 @@ __device__ __forceinline__ void grad_row_general(const GradP &p, const GradRow &
 
 template <int DT, int MK, bool KL, int GDT, bool AL>
 __global__ __launch_bounds__(kGradThreads) void k_score_grad(GradP p) {
-    const int64_t row = blockIdx.x / unsigned(p.parts);
-    const int part = int(blockIdx.x % unsigned(p.parts));
+    int64_t row = blockIdx.x;
+    int part = 0;
+    if (p.parts > 1) {
+        row = blockIdx.x / unsigned(p.parts);
+        part = int(blockIdx.x % unsigned(p.parts));
+    }
     const GradRow g = grad_row<KL>(p, row);
     if (p.tau_one) {
         if constexpr (AL) grad_row_aligned<DT, MK, KL, GDT, true>(p, g, row, part);
