@@ -9,11 +9,11 @@
 // Each element becomes one 64-bit key, (order key << 32) | ~position, so that a plain descending
 // comparison of keys is CpuRef's order with ties broken by position, and no two keys are equal.
 // A lane of up to kSortCap elements is sorted by one workgroup (four counting passes over the order
-// key in LDS). A longer lane is
-// cut into kSortCap-long runs, each sorted that way into a scratch buffer, and the runs are
-// merged pairwise (merge path: each workgroup stages the two input windows that feed its tile of
-// outputs into LDS and merges them there) until one run remains. The last step writes each position's value, decoded from its key (a NaN is read back
-// from its source to keep the payload), and its index.
+// key in LDS). A longer lane is cut into runs of kSortCap, or of a quarter of it where few lanes
+// leave CUs idle, each sorted that way into a scratch buffer, and the runs are merged pairwise
+// (merge path: each workgroup stages the two input windows that feed its tile of outputs into LDS
+// and merges them there) until one run remains. The last step writes each position's value,
+// decoded from its key (a NaN is read back from its source to keep the payload), and its index.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -30,7 +30,7 @@ namespace {
 constexpr int kSortCap = 16384;  // elements one workgroup sorts in LDS (the longest run)
 constexpr int kMergeThreads = 256;
 constexpr int kMergeItems = 8;   // outputs per thread of a merge pass
-constexpr int kMergeTile = kMergeThreads * kMergeItems;  // outputs per workgroup (divides 2 kSortCap)
+constexpr int kMergeTile = kMergeThreads * kMergeItems;  // outputs per workgroup (divides twice a run)
 constexpr int kWaveSize = 64;
 
 // CpuRef's order as an unsigned key: every NaN, whatever its sign and payload, above +inf, then
@@ -58,6 +58,8 @@ struct SortP {
     uint64_t *runs;   // [lanes][n] sorted runs (multi-run lanes)
     int64_t outer, n, inner;
     int32_t chunks;   // runs per lane
+    int32_t run;      // elements per run
+    int32_t wide;     // merges find their co-ranks with a wave each
 };
 
 // Sort run `chunk` of lane `lane` (at most THREADS x E elements) by four stable counting passes over
@@ -83,7 +85,7 @@ __global__ __launch_bounds__(THREADS) void k_sort_runs(SortP p) {
     const int64_t lane_id = blockIdx.x / p.chunks;
     const int chunk = int(blockIdx.x - lane_id * p.chunks);
     const int64_t o = lane_id / p.inner, i = lane_id - o * p.inner;
-    const int64_t beg = int64_t(chunk) * kSortCap;
+    const int64_t beg = int64_t(chunk) * p.run;
     const int len = int(std::min<int64_t>(CAP, p.n - beg));
     const int tid = threadIdx.x, lane = tid % kWaveSize, w = tid / kWaveSize;
     const int t0 = w * kWaveSize * E + lane;  // element of register 0
@@ -171,12 +173,28 @@ __global__ __launch_bounds__(THREADS) void k_sort_runs(SortP p) {
     }
 }
 
+// Elements per run. A lane that one workgroup can hold is one run. Longer lanes whose runs of kSortCap
+// would leave most CUs idle are cut four times finer: the runs are bound by one workgroup's time, and two
+// more merge passes (8.5 us each) cost less than it saves. Measured (us, runs of 16384 and halving co-ranks /
+// this rule): 1 row of 32000 57.1 / 40.9, 1 of 128256 80.9 / 59.0, 8 of 50257 70.4 / 56.1, 8 of 128256 (64
+// runs) 95.0 / 85.8; from there on the two meet (16 of 128256 keep runs of 16384, 102.5).
+int32_t sort_run(int64_t lanes, int64_t n) {
+    if (n <= kSortCap) return kSortCap;
+    return lanes * ((n + kSortCap - 1) / kSortCap) <= 64 ? kSortCap / 4 : kSortCap;
+}
+
+// Up to this many workgroups a merge pass waits for its co-ranks' dependent loads, past it for the loads'
+// number: a pass over [1, 128256] takes 8.5 us with a wave's co-ranks and 12 by halving, over
+// [64, 128256] (4032 workgroups) 44.6 and 35.9.
+constexpr int64_t kWideMerges = 512;
+
 // Threads and elements per thread for runs of up to `longest` elements: the smallest that hold them.
 void launch_runs(const SortP &p, int64_t longest, int64_t blocks, hipStream_t s) {
     const dim3 grid{unsigned(blocks)};
     if (longest <= 256) hipLaunchKernelGGL((k_sort_runs<256, 1>), grid, dim3(256), 0, s, p);
     else if (longest <= 1024) hipLaunchKernelGGL((k_sort_runs<256, 4>), grid, dim3(256), 0, s, p);
-    else if (longest <= 4096) hipLaunchKernelGGL((k_sort_runs<256, 16>), grid, dim3(256), 0, s, p);
+    else if (longest <= 4096 && p.chunks == 1) hipLaunchKernelGGL((k_sort_runs<256, 16>), grid, dim3(256), 0, s, p);
+    else if (longest <= 4096) hipLaunchKernelGGL((k_sort_runs<1024, 4>), grid, dim3(1024), 0, s, p);
     else if (longest <= 8192) hipLaunchKernelGGL((k_sort_runs<1024, 8>), grid, dim3(1024), 0, s, p);
     else hipLaunchKernelGGL((k_sort_runs<1024, 16>), grid, dim3(1024), 0, s, p);
 }
@@ -189,6 +207,21 @@ __device__ __forceinline__ int64_t co_rank(const uint64_t *A, int64_t la, const 
         const int64_t mid = (lo + hi) >> 1;
         if (A[mid] > B[d - mid - 1]) lo = mid + 1;
         else hi = mid;
+    }
+    return lo;
+}
+
+// The same by one wave: its lanes probe 64 ascending points of the range at once, three rounds of
+// dependent loads for runs of 65536 where halving takes 17.
+__device__ __forceinline__ int64_t co_rank_wave(const uint64_t *A, int64_t la, const uint64_t *B, int64_t lb, int64_t d) {
+    const int lane = threadIdx.x % kWaveSize;
+    int64_t lo = std::max<int64_t>(0, d - lb), hi = std::min<int64_t>(d, la);
+    while (lo < hi) {
+        const int64_t span = hi - lo, mid = lo + span * lane / kWaveSize;  // in [lo, hi - 1]
+        const int t = __builtin_popcountll(__ballot(A[mid] > B[d - mid - 1]));  // true up to the answer
+        const int64_t l = lo;
+        if (t > 0) lo = l + span * (t - 1) / kWaveSize + 1;
+        if (t < kWaveSize) hi = l + span * t / kWaveSize;
     }
     return lo;
 }
@@ -217,7 +250,15 @@ __global__ __launch_bounds__(kMergeThreads) void k_merge(SortP p, const uint64_t
     const uint64_t *A = src + lane * n + base;
     const uint64_t *B = A + la;
     const int64_t d0 = o0 - base, d1 = o1 - base;
-    if (tid < 2) cr[tid] = co_rank(A, la, B, lb, tid == 0 ? d0 : d1);
+    if (p.wide) {
+        const int wave = tid / kWaveSize;
+        if (wave < 2) {
+            const int64_t c = co_rank_wave(A, la, B, lb, wave == 0 ? d0 : d1);
+            if (tid % kWaveSize == 0) cr[wave] = c;
+        }
+    } else if (tid < 2) {
+        cr[tid] = co_rank(A, la, B, lb, tid == 0 ? d0 : d1);
+    }
     __syncthreads();
     const int64_t a0 = cr[0], b0 = d0 - cr[0];
     const int na = int(cr[1] - cr[0]), nb = int((d1 - cr[1]) - b0);
@@ -289,7 +330,8 @@ int nt_hip_sort_desc(const float *x, int64_t outer, int64_t n, int64_t inner, fl
     p.outer = outer;
     p.n = n;
     p.inner = inner;
-    const int64_t chunks = (n + kSortCap - 1) / kSortCap;
+    p.run = sort_run(lanes, n);
+    const int64_t chunks = (n + p.run - 1) / p.run;
     if (lanes * chunks > int64_t(0x7fffffff)) return fail(NT_E_ARG, "sort_desc: too many lanes");
     p.chunks = int32_t(chunks);
     std::unique_lock<std::mutex> lk;
@@ -307,17 +349,18 @@ int nt_hip_sort_desc(const float *x, int64_t outer, int64_t n, int64_t inner, fl
         return rc;
     }
     p.runs = static_cast<uint64_t *>(buf[0]);
-    launch_runs(p, kSortCap, lanes * chunks, st);
+    launch_runs(p, p.run, lanes * chunks, st);
     int rc = launched("k_sort_runs");
     const int64_t tiles = (n + kMergeTile - 1) / kMergeTile;
     const int64_t blocks = lanes * tiles;
+    p.wide = blocks <= kWideMerges;
     if (blocks > int64_t(0x7fffffff)) {
         scratch_release(buf[0]);
         scratch_release(buf[1]);
         return fail(NT_E_ARG, "sort_desc: too many merge tiles");
     }
     int cur = 0;
-    for (int64_t w = kSortCap; !rc && w < n; w *= 2) {
+    for (int64_t w = p.run; !rc && w < n; w *= 2) {
         const uint64_t *src = static_cast<const uint64_t *>(buf[cur]);
         uint64_t *dst = static_cast<uint64_t *>(buf[cur ^ 1]);
         if (2 * w >= n) {

@@ -39,3 +39,16 @@ def test_values_and_positions(n, kind):
     wv, wi = T.sort_desc(x, list(x.shape), 1)
     np.testing.assert_array_equal(i.to_numpy(), wi)
     np.testing.assert_array_equal(v.to_numpy().view(np.uint32), np.asarray(wv, F).view(np.uint32))
+
+
+# the number of lanes also chooses the run's length (up to 64 long runs: a quarter) and the co-ranks'
+# search (up to 512 merge tiles: a wave each): both sides of both, with partial last runs and tiles
+@pytest.mark.parametrize("shape", [(32, 16385, 1), (33, 16385, 1), (1, 70001, 1), (64, 16389, 1), (8, 20480, 3),
+                                   (29, 36865, 1)])
+@pytest.mark.parametrize("kind", ["ties", "bits"])
+def test_lane_counts(shape, kind):
+    x = lanes(kind, shape, shape[1])
+    v, i = ops.sort_desc(nr.Tensor.from_numpy(x), shape)
+    wv, wi = T.sort_desc(x, list(shape), 1)
+    np.testing.assert_array_equal(i.to_numpy(), wi)
+    np.testing.assert_array_equal(v.to_numpy().view(np.uint32), np.asarray(wv, F).view(np.uint32))
