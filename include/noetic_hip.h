@@ -98,7 +98,8 @@ int nt_hip_platform_details(char *buf, size_t cap);
  * nt_hip_alloc takes memory from the device's stream-ordered pool when it has one: it is valid for
  * work queued on the library stream after the call. nt_hip_free only records the pointer and
  * returns at once (the reference's Mem drop, src/tensor/cuda/backend.rs:35-45); the next entry
- * point frees it on the stream, after the work queued before the release. */
+ * point keeps it for a later allocation of its size class (bounded; everything runs on the one
+ * stream) or frees it on the stream, after the work queued before the release. */
 int nt_hip_alloc(size_t bytes, void **out);
 int nt_hip_free(void *ptr);
 int nt_hip_upload(void *dst, const void *src, size_t bytes);   /* host -> device, synchronous */

@@ -23,7 +23,7 @@
 // A half product (GpuBackend::matmul_half; HALF) takes the same path: panels of 64 k rounded to bf16 on
 // their way into LDS, 16 k per v_mfma_f32_32x32x16_bf16, one accumulator over the whole of k.
 // Against the kernel before it, whose loads were branches between whole, unaligned and last panels:
-// 1024^3 24.2 -> 12.6 us, 247 x 525 x 914 39.9 -> 9.1, 300 x 3000 x 3000 391 -> 38.7, 2048^3 59.1 -> 35.7.
+// 1024^3 24.2 -> 12.6 us, 247 x 525 x 914 39.9 -> 9.1, 300 x 3000 x 3000 391 -> 38.7, 2048^3 59.1 -> 38.4.
 //
 // Workgroups are renumbered so that each of the 8 XCDs (which the hardware deals consecutive
 // workgroups to in turn) works on a contiguous run of tiles, whose A panels then stay in that
