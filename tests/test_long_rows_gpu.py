@@ -56,6 +56,27 @@ def test_first_maximum_of_long_rows(n):
     np.testing.assert_array_equal(ops.reduce_dim(ReduceOp.ARGMAX, t, (6, n), 1).to_numpy().ravel(), x.argmax(1))
 
 
+# a wave per row from 1024 rows of up to 4096, and from 4096 of up to 8192: both sides of each line, and
+# rows shorter than a wave and than its eight loads
+@pytest.mark.parametrize("rows,n", [(1024, 1), (1025, 63), (1027, 65), (1024, 511), (1023, 513), (1024, 4096), (1030, 4097),
+                                    (4096, 8191), (4099, 8193), (70001, 9)])
+def test_first_maximum_of_many_rows(rows, n):
+    rng = np.random.default_rng(rows + n)
+    x = rng.integers(-50, 50, (rows, n)).astype(F)  # ties
+    x[1, n // 3] = np.nan
+    x[2, n // 2:] = np.nan
+    x[3] = -np.inf
+    x[5, -1] = np.inf
+    x[rows - 1, -1] = np.nan
+    x[6], x[7] = 0.0, -0.0
+    x[6, n // 2:] = -0.0  # equal zeros: the first one, sign and all
+    t = nr.Tensor.from_numpy(x)
+    at = x.argmax(1)
+    np.testing.assert_array_equal(ops.reduce_dim(ReduceOp.ARGMAX, t, (rows, n), 1).to_numpy().ravel(), at)
+    np.testing.assert_array_equal(ops.reduce_dim(ReduceOp.MAX, t, (rows, n), 1).to_numpy().ravel().view(np.uint32),
+                                  x[np.arange(rows), at].view(np.uint32))
+
+
 @pytest.mark.parametrize("op", list(BinaryOp))
 @pytest.mark.parametrize("rows,cols,off", [(1, 1024, 0), (3, 1023, 0), (3, 1024, 0), (4, 4097, 0), (2, 5000, 1),
                                            (40000, 1028, 0)])
