@@ -155,7 +155,8 @@ extern "C" int nt_hip_rl_sample_gumbel(const NtRlGumbelArgs *a) {
     p.vec = reinterpret_cast<uintptr_t>(a->logits) % 16 == 0 && (a->ld * esz) % 16 == 0 && mask_vec && V % 8 == 0 &&
             V * 4 <= int64_t(0x7fffffff);
     p.inv_tau = p.tau_one || a->mask_kind == NT_MASK_F32 ? 1.0f : 1.0f / p.tau;
-    p.m_ovf = p.tau_one || a->mask_kind == NT_MASK_F32 ? -INFINITY : neg_overflow_bound(p.tau);
+    // (an infinite factor would take every negative logit's bound to -inf, whatever its quotient)
+    if (!std::isfinite(p.inv_tau)) p.inv_tau = NAN;
     p.col = chacha_columns(p.key);
     hipStream_t s = ctx().stream;
     const int64_t nblk = V / 8 + 2;

@@ -20,8 +20,8 @@ struct GumbelP {
     MaskMap mm;  // the mask row of each logits row
     float tau;
     int tau_one;
-    float inv_tau;  // 1 / tau in f32 (1 at tau == 1, and under an additive mask: its values are divided)
-    float m_ovf;    // the largest logit whose quotient by tau is -inf (neg_overflow_bound; -inf likewise)
+    float inv_tau;  // 1 / tau in f32 (1 at tau == 1, and under an additive mask: its values are divided); NaN
+                    // where it overflows, up to tau = 2^-128: no bound then skips an element
     ChachaKey key;
     ChachaColumns col;
     uint64_t h;  // pair index of the stream's u64 0: its low word is keystream word 2 h + ODD
@@ -223,7 +223,8 @@ __device__ __forceinline__ float gumbel_bound(uint32_t hi) {
 
 // What a bound must reach to be looked at, beside a largest screened value x so far: screen_floor, less
 // the bound's slack and the rounding of x inv_tau (and no more than 3e38, so that a logit whose
-// rounded product is finite where its quotient is infinite is looked at too).
+// rounded product is finite where its quotient is infinite is looked at too). A NaN bound reaches
+// every floor: with inv_tau NaN each element is divided and screened.
 __device__ __forceinline__ float bound_floor(float x) {
     return fminf(screen_floor(x, 0x1p-20f) - fmaxf(2.0f * kGumbelScreen, fabsf(x) * 0x1p-20f), 3e38f);
 }
@@ -596,12 +597,12 @@ __global__ __launch_bounds__(kGumbelMaxThreads) void k_sample_gumbel(GumbelP p) 
             for (int j = 0; j < 8; j++) look |= !(bound[j] < near) && have ? 1u << j : 0u;
             bool moved = false;
             g.each(look, x, wlo, whi, [&](int j, float xj, uint32_t lj, uint32_t hj) {
-                if (xj <= p.m_ovf) return;  // excluded, or its quotient by tau is -inf
-                if (xj != xj) {
+                const float z = MK == NT_MASK_F32 || p.tau_one ? xj : xj / p.tau;
+                if (z == -INFINITY) return;  // excluded, or its quotient by tau is -inf
+                if (z != z) {  // (0 / 0 too, where tau is 0 in f32)
                     g.flags |= 2;
                     return;
                 }
-                const float z = MK == NT_MASK_F32 || p.tau_one ? xj : xj / p.tau;
                 g.flags |= 1;
                 const float a = z + gumbel_screen(lj, hj);
                 moved |= a > amax;

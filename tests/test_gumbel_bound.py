@@ -3,6 +3,7 @@ is never below the draw's g = -ln(-ln u) by more than the slack of bound_floor (
 what is sure), and above it by at most 1e-3 except at the ends of the range, where what is sure is not taken
 from it. numpy's f32 logarithm stands in for the hardware's (both within about an ulp)."""
 import numpy as np
+import pytest
 
 
 def bound(hi):
@@ -33,3 +34,29 @@ def test_bound_over_the_range_of_the_high_word():
         sure = (hi >= np.uint32(0x1000)) & (hi < np.uint32(0xFFFF0000))
         assert np.all(b[sure] <= g[sure] + 1e-3)
     assert bound(np.array([0xFFFFFFFF], np.uint32))[0] == np.inf
+
+
+# The bound with the logit's share: x inv_tau + bound(hi), inv_tau NaN where 1 / tau overflows in f32 (the
+# host's rule). An element may be skipped only where its bound is below bound_floor of its own value:
+# below any floor that a larger one sets.
+@pytest.mark.parametrize("tau", [0.0, 1e-45, 1e-40, 2.9387e-39, 2.9388e-39, 1e-37, 1e-20, 0.6, 3.0, 1e20, 3e38])
+def test_no_element_is_skipped_beside_itself(tau):
+    f = np.float32
+    rng = np.random.default_rng(2)
+    tau = f(tau)
+    hi = rng.integers(1 << 16, (1 << 32) - (1 << 16), 200_000, dtype=np.uint64).astype(np.uint32)
+    x = (rng.normal(0, 3, hi.size) * 10.0 ** rng.uniform(-44, 30, hi.size)).astype(f)
+    x[:1000] = 0.0
+    with np.errstate(all="ignore"):
+        near_one = (rng.normal(0, 3, hi.size).astype(f) * tau).astype(f)  # quotients of a logit's size
+        x[1000:100_000] = near_one[1000:100_000]
+        inv = f(1) / tau
+        if not np.isfinite(inv):
+            inv = f(np.nan)
+        z = (x / tau).astype(f)
+        a = (z + g_of(hi, np.zeros_like(hi)).astype(f)).astype(f)
+        b = (x * inv + bound(hi)).astype(f)
+        screen = a - np.maximum(f(1e-3), np.abs(a) * f(2.0 ** -20))
+        floor = np.fmin(screen - np.maximum(f(2e-3), np.abs(a) * f(2.0 ** -20)), f(3e38))
+    candidate = ~np.isnan(z) & (z > -np.inf)
+    assert not np.any(candidate & (b < floor))

@@ -79,6 +79,43 @@ def test_ties_and_full_slots_over_segments(value, tau):
     np.testing.assert_array_equal(dev, cpu)
 
 
+@pytest.mark.parametrize("tau", [1e-45, 1e-40, 2.9e-39, 3e-39])
+@pytest.mark.parametrize("rows,mask", [(260, None), (260, "u8"), (2, None)])
+def test_temperatures_whose_reciprocal_overflows(tau, rows, mask):
+    """Logits of the temperature's own size, several steps of each wave: their quotients are ordinary
+    values although x (1 / tau) is infinite, and zeros' quotients are zeros."""
+    V = 20000 if rows > 2 else 700_000
+    rng = np.random.default_rng(rows)
+    x = (rng.normal(-2, 2, (rows, V)) * tau).astype(F)
+    x[1] = np.minimum(x[1], -F(1e-45))
+    x[0, 5:] = 0.0
+    if rows > 2:
+        x[3] = -0.1  # quotients near -1e38 or -inf, and one row of them beside a zero in its last block
+        x[3, V - 1] = 0.0
+        x[4] = np.where(np.arange(V) % 7 == 0, F(0.25), x[4])  # overflows to +inf: the first of them
+    keep = None
+    if mask:
+        keep = (rng.random((rows, V)) < 0.5).astype(np.uint8)
+        keep[:, V - 1] = 1
+    dev, cpu = both(x, tau, 17, keep=keep)
+    np.testing.assert_array_equal(dev, cpu)
+
+
+def test_a_temperature_that_is_zero_in_f32():
+    """T = 1e-46 divides by an f32 zero: +inf for a positive logit, -inf for a negative one, a NaN (refused)
+    for a zero."""
+    x = np.full((3, 9000), -1.0, F)
+    x[:, 8000] = x[:, 8500] = 2.0
+    dev, cpu = both(x, 1e-46, 5)
+    np.testing.assert_array_equal(dev, cpu)
+    assert (dev == 8000).all()
+    for value in (0.0, -2.0):  # row 1: 0 / 0, or nothing above -inf
+        y = x.copy()
+        y[1, 8000] = y[1, 8500] = value
+        with pytest.raises(ValueError, match="position 1 has no allowed token"):
+            both(y, 1e-46, 5)
+
+
 def test_reruns_and_more_rows_agree():
     """A row's token does not depend on how the launch was cut: the first rows of a launch of 300 (one
     workgroup each) against the same rows alone."""
