@@ -521,6 +521,37 @@ __device__ __forceinline__ float row_sum_dpp(float v) {
     v = v + dpp_mov<0x140>(v);
     return v;
 }
+// f of the four rows' lanes of one column, in a fixed order (gfx950's swaps of rows and of halves).
+template <class F>
+__device__ __forceinline__ float across_rows(float v, F f) {
+    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = f(__uint_as_float(p[0]), __uint_as_float(p[1]));
+    const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return f(__uint_as_float(q[0]), __uint_as_float(q[1]));
+}
+
+// N values folded over the 64 lanes at once (N 1, 2 or 4): lane k holds value k's fold, lanes exchanging
+// the values that are not theirs in the first steps. Fixed orders throughout.
+template <int N, class F>
+__device__ __forceinline__ float wave_folds(const float (&x)[N], F f) {
+    const int lane = int(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)));
+    const bool b0 = lane & 1, b1 = lane & 2;
+    float v;
+    if constexpr (N == 1) {
+        v = f(x[0], dpp_mov<0xB1>(x[0]));
+        v = f(v, dpp_mov<0x4E>(v));
+    } else if constexpr (N == 2) {
+        v = f(b0 ? x[1] : x[0], dpp_mov<0xB1>(b0 ? x[0] : x[1]));
+        v = f(v, dpp_mov<0x4E>(v));
+    } else {
+        const float s = f(b0 ? x[1] : x[0], dpp_mov<0xB1>(b0 ? x[0] : x[1]));
+        const float t = f(b0 ? x[3] : x[2], dpp_mov<0xB1>(b0 ? x[2] : x[3]));
+        v = f(b1 ? t : s, dpp_mov<0x4E>(b1 ? s : t));
+    }
+    v = f(v, dpp_mov<0x124>(v));  // row_ror:4 and :8
+    v = f(v, dpp_mov<0x128>(v));
+    return across_rows(v, f);
+}
 __device__ __forceinline__ int wave_min_i(int v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, kWave));

@@ -12,8 +12,8 @@
 //  * Arithmetic: f32 per element; bf16 is widened exactly by a shift. Exponentials are
 //    exp2 of (v - shift) * c on the hardware v_exp_f32, where c = log2(e) / temperature folds
 //    the temperature divide into the exponent (no per-element divide).
-//  * Determinism: no atomics; every reduction (per lane, across a wave, across waves) has a
-//    fixed order independent of timing, so reruns are bit-identical (the contract of
+//  * Determinism: every reduction (per lane, across a wave, across waves) has a fixed order
+//    independent of timing, so reruns are bit-identical (the contract of
 //    src/nn/tests/gpu/rl.rs:125-128).
 //
 // Sampler (nt_hip_rl_sample): each chunk's (max, sum of exp) goes to LDS; wave 0 then merges
@@ -21,10 +21,10 @@
 // (512 elements, an L2 hit in practice) and scans it in f64. HBM traffic is one pass over the
 // row plus one chunk.
 //
-// Scorer (nt_hip_rl_score): every lane keeps running (max, sum exp, sum exp*d, sum exp*(z-r))
-// for the policy and (max, sum exp) for the reference, rescaled when its max grows (online
-// log-sum-exp); waves and then the workgroup merge them in a fixed order; per-row scalars are
-// finished in f64.
+// Scorer (nt_hip_rl_score): every batch of chunks becomes a record (max, sum exp, sum exp*d,
+// sum exp*(z-r)) for the policy and (max, sum exp) for the reference, summed over the wave in f32
+// relative to the batch's maxima; a row's records are merged in a fixed order, and its scalars
+// finished, in f64. How a row is cut depends on the vocabulary and the mask's kind alone.
 #include <algorithm>
 
 #include "nt_launch.hpp"
@@ -268,33 +268,46 @@ __global__ void k_kl_estimate_grad(const float *lp, const float *lr, const float
 
 // ------------------------------------------------------------------ dispatch helpers
 
-// The states of a launch with several workgroups per row. Every such launch is on the library's one
+// The records of a launch with several workgroups per row. Every such launch is on the library's one
 // stream (a launch under capture takes one workgroup per row: its graph may be replayed on another).
-constexpr int kScorePartStates = 1024;
-__device__ RowState g_score_part[kScorePartStates];
+constexpr int kScoreSplitRows = 256;
+__device__ RowRec g_score_part[kScoreSplitRows * kScoreRecs];
 
 // This device's address of g_score_part (the host-side name is only a stand-in).
-int score_parts(RowState **out) {
-    static RowState *at = nullptr;  // (one device per process; the context's lock is held)
+int score_parts(RowRec **out) {
+    static RowRec *at = nullptr;  // (one device per process; the context's lock is held)
     if (!at) {
         void *ptr = nullptr;
         if (int rc = hip_check(hipGetSymbolAddress(&ptr, HIP_SYMBOL(g_score_part)), "hipGetSymbolAddress")) return rc;
-        at = static_cast<RowState *>(ptr);
+        at = static_cast<RowRec *>(ptr);
     }
     *out = at;
     return 0;
 }
 
-// Workgroups per row of the scorer: one CU reads a row at about 10 GB/s per KiB in flight, so few rows
-// leave the chip idle. About 1024 workgroups, each of at least 8 chunks (two per wave in flight
-// at once), or 24 past 64 rows, where the finishing launch (2.5 us) weighs more. Measured (us, one
-// workgroup per row / this rule): 1 row of 128256 bf16 23.7 / 7.3, 16 of 151936 with a reference
-// 42.3 / 12.0, 64 of 128256 under a shared f32 mask 32.6 / 12.6, 120 of 50304 f32 18.6 / 12.6, 256 of
-// 128256 with a u8 mask 30.5 / 23.1; two workgroups per row of 400 x 32000 lost, 13.0 / 16.1.
-int score_segs(int64_t rows, int nc) {
-    if (rows > 256) return 1;
-    const int64_t g = std::min<int64_t>(kScorePartStates / rows, nc / (rows <= 64 ? 8 : 24));
-    return int(std::min<int64_t>(std::max<int64_t>(g, 1), kScoreMaxSegs));
+// Chunks per batch of rows of nc chunks, at most: what a wave holds decoded beside the next batch's loads.
+int score_batch(int nc, int mk) { return mk == NT_MASK_F32 || nc <= 32 ? 2 : 4; }
+
+// How a row of nc chunks is cut, from the vocabulary and the mask's kind alone (the row's bits depend on
+// it): batches of fewer chunks where four waves would not have one each, and as many batches per record as
+// kScoreRecs asks for.
+void score_cut(int nc, int mk, ScoreP *p) {
+    p->nc = nc;
+    p->batch = std::min(score_batch(nc, mk), (nc + kScoreWaves - 1) / kScoreWaves);
+    const int n = (nc + p->batch - 1) / p->batch;
+    p->per = (n + kScoreRecs - 1) / kScoreRecs;
+    p->recs = (n + p->per - 1) / p->per;
+}
+
+// Workgroups per row of the scorer: few rows leave the chip idle. About 1024 workgroups, each of at
+// least a record per wave, or 24 chunks past 64 rows, where the finishing launch (2.5 us) weighs more;
+// 768 with a reference, of which three fit a CU. Rows of fewer than 40 chunks are not worth that launch.
+// Measured (us, one workgroup per row / this rule): 1 row of 128256 bf16 20.4 / 6.5, 64 of 128256 under an
+// f32 mask with a reference 52.4 / 18.1, 256 of 128256 with a u8 mask 37.6 / 29.9; 1 of 8200 5.1 / 6.2 if split.
+int score_segs(int64_t rows, const ScoreP &p, bool ref) {
+    if (rows > kScoreSplitRows || p.nc < 40) return 1;
+    const int most = rows <= 64 ? (p.recs + kScoreWaves - 1) / kScoreWaves : p.nc / 24;
+    return std::max(1, std::min((ref && rows > 64 ? 768 : 1024) / int(rows), most));
 }
 
 // Workgroups per row of the backward (their steps are independent): about 4096, each of two steps or
@@ -308,11 +321,22 @@ int grad_parts(int64_t rows, int64_t vocab) {
 template <int DT, int MK, bool REF, bool KL, bool ENT>
 void pick_al_score(bool al, const ScoreP &p, int64_t rows, hipStream_t s) {
     char nm[96];
-    std::snprintf(nm, sizeof nm, "nt::k_score<%d, %d, %s, %s, %s, %s>", DT, MK, rtc_bool(REF), rtc_bool(KL),
-                  rtc_bool(ENT), rtc_bool(al));
     const dim3 grid(unsigned(rows * p.segs));
-    if (al) launch_path(k_score<DT, MK, REF, KL, ENT, true>, nm, grid, dim3(kScoreThreads), 0, s, p);
-    else launch_path(k_score<DT, MK, REF, KL, ENT, false>, nm, grid, dim3(kScoreThreads), 0, s, p);
+    auto launch = [&](auto alc, auto nbc) {
+        constexpr bool AL = decltype(alc)::value;
+        constexpr int NB = decltype(nbc)::value;
+        std::snprintf(nm, sizeof nm, "nt::k_score<%d, %d, %s, %s, %s, %s, %d>", DT, MK, rtc_bool(REF), rtc_bool(KL),
+                      rtc_bool(ENT), rtc_bool(AL), NB);
+        launch_path(k_score<DT, MK, REF, KL, ENT, AL, NB>, nm, grid, dim3(kScoreThreads), 0, s, p);
+    };
+    auto by_nb = [&](auto alc) {
+        if constexpr (MK != NT_MASK_F32) {
+            if (score_batch(p.nc, MK) == 4) return launch(alc, std::integral_constant<int, 4>{});
+        }
+        launch(alc, std::integral_constant<int, 2>{});
+    };
+    if (al) by_nb(std::true_type{});
+    else by_nb(std::false_type{});
     if (p.segs > 1) {
         std::snprintf(nm, sizeof nm, "nt::k_score_finish<%d, %d, %s, %s, %s>", DT, MK, rtc_bool(REF), rtc_bool(KL),
                       rtc_bool(ENT));
@@ -374,7 +398,7 @@ int nt_hip_rl_score(const NtRlScoreArgs *a) {
     p.tau = float(a->temperature);
     p.tau_one = (a->temperature == 1.0);
     p.c = (a->mask_kind == NT_MASK_F32 || p.tau_one) ? kLog2e : float(double(kLog2e) / double(p.tau));
-    p.nc = int((a->vocab + kChunk - 1) / kChunk);
+    score_cut(int((a->vocab + kChunk - 1) / kChunk), a->mask_kind, &p);
     p.tokens = a->tokens;
     p.logp = a->logp;
     p.ref_logp = a->ref_logp;
@@ -393,7 +417,7 @@ int nt_hip_rl_score(const NtRlScoreArgs *a) {
               a->vocab * 4 <= int64_t(0x7fffffff);
     if (ref) al = al && reinterpret_cast<uintptr_t>(a->ref_logits) % 16 == 0;
     hipStream_t s = ctx().stream;
-    p.segs = score_segs(a->rows, p.nc);
+    p.segs = score_segs(a->rows, p, ref);
     p.part = nullptr;
     if (p.segs > 1) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;

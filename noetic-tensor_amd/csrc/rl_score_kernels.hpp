@@ -28,62 +28,61 @@ struct ScoreP {
     float *logp, *ref_logp, *kl, *ent;
     uint8_t *status;
     float *lse_base, *lse_rest, *ref_lse_base, *ref_lse_rest;
-    int segs;               // workgroups per row
-    struct RowState *part;  // segs > 1: their states, [rows][segs]
+    int batch;            // chunks per batch (at most the kernel's NB)
+    int per;              // batches per record
+    int recs;             // records per row
+    int segs;             // workgroups per row
+    struct RowRec *part;  // segs > 1: the records, [rows][recs]
 };
 
-// Running state of one lane (value space, exponent scale c). Every sum is relative to the
-// lane's running maxima, so no term cancels against another of size |logit|:
+// What a wave found in a run of chunks (value space, exponent scale c). Every sum is relative to the
+// run's own maxima, so no term cancels against another of size |logit|:
 //   S  = sum w,                 w = exp2((v - a) c)
 //   H  = sum w (v - a) c                                  (entropy)
 //   B  = sum w ((v - a) - (v_ref - a_ref)) c              (exact KL)
 //   Sr = sum exp2((v_ref - a_ref) c)                      (reference normaliser)
-struct RowState {
+struct RowRec {
     float a, S, H, B;
     float ar, Sr;
 };
 
+// Sums in f64 relative to the maxima af and arf.
+struct RowSums {
+    double S, H, B, Sr;
+};
+
 __device__ __forceinline__ float shift_of(float a) { return a == -INFINITY ? 0.0f : a; }
 
-// The B update when the maxima move by d = (a_old - a_new) c and e = (a_ref_old - a_ref_new) c:
-// B' = f (B + (d - e) S). A state with S == 0 holds no policy term.
-__device__ __forceinline__ float b_rescaled(float B, float S, float f, float d, float e) {
-    return S > 0.0f ? f * (B + (d - e) * S) : 0.0f;
-}
-
-// Merge state o into s (the same arithmetic whichever side is s).
+// Record r's sums, moved to the maxima af and arf (at least its own), added to t.
 template <bool REF, bool KL, bool ENT>
-__device__ __forceinline__ void state_merge(RowState &s, const RowState &o, float c) {
-    const float an = fmaxf(s.a, o.a), sh = shift_of(an);
-    const float d1 = (s.a - sh) * c, d2 = (o.a - sh) * c;
-    const float f1 = exp2_hw(d1), f2 = exp2_hw(d2);
-    float e1 = 0.0f, e2 = 0.0f;
-    if constexpr (REF) {
-        const float anr = fmaxf(s.ar, o.ar), shr = shift_of(anr);
-        e1 = (s.ar - shr) * c;
-        e2 = (o.ar - shr) * c;
-        s.Sr = exp2_hw(e1) * s.Sr + exp2_hw(e2) * o.Sr;
-        s.ar = anr;
+__device__ __forceinline__ void rec_add(RowSums &t, const RowRec &r, float af, float arf, float c) {
+    if (r.S > 0.0f) {
+        const double d = (double(r.a) - double(af)) * double(c), f = exp2(d);
+        t.S += f * double(r.S);
+        if constexpr (ENT) t.H += f * (double(r.H) + d * double(r.S));
+        if constexpr (KL) {
+            const double e = (double(r.ar) - double(arf)) * double(c);
+            t.B += f * (double(r.B) + (d - e) * double(r.S));
+        }
+    } else if (!(r.S == r.S)) {
+        t.S = NAN;
     }
-    if constexpr (ENT) s.H = f1 * (s.H + fmaxf(d1, -FLT_MAX) * s.S) + f2 * (o.H + fmaxf(d2, -FLT_MAX) * o.S);
-    if constexpr (KL) s.B = b_rescaled(s.B, s.S, f1, d1, e1) + b_rescaled(o.B, o.S, f2, d2, e2);
-    s.S = f1 * s.S + f2 * o.S;
-    s.a = an;
+    if (REF && r.ar != -INFINITY) t.Sr += exp2((double(r.ar) - double(arf)) * double(c)) * double(r.Sr);
 }
 
-__device__ __forceinline__ RowState shfl_down_state(const RowState &s, int o) {
-    RowState r;
-    r.a = __shfl_down(s.a, o, kWave);
-    r.S = __shfl_down(s.S, o, kWave);
-    r.H = __shfl_down(s.H, o, kWave);
-    r.B = __shfl_down(s.B, o, kWave);
-    r.ar = __shfl_down(s.ar, o, kWave);
-    r.Sr = __shfl_down(s.Sr, o, kWave);
-    return r;
+// Record o added to s (rows of more than kScoreRecs batches: a record then holds several).
+template <bool REF, bool KL, bool ENT>
+__device__ __forceinline__ void rec_merge(RowRec &s, const RowRec &o, float c) {
+    const float a = fmaxf(s.a, o.a), ar = fmaxf(s.ar, o.ar);
+    RowSums t{0.0, 0.0, 0.0, 0.0};
+    rec_add<REF, KL, ENT>(t, s, a, ar, c);
+    rec_add<REF, KL, ENT>(t, o, a, ar, c);
+    s = RowRec{a, float(t.S), float(t.H), float(t.B), ar, float(t.Sr)};
 }
 
 constexpr int kScoreThreads = 256;
 constexpr int kScoreWaves = kScoreThreads / kWave;
+constexpr int kScoreRecs = 256;  // records per row, at most
 
 // load_raw for aligned rows through per-row buffer resources (row bytes below 2^31), no bounds
 // branch, 32-bit offsets, non-temporal (every input is read once). Past the row's end the
@@ -201,11 +200,47 @@ __device__ __forceinline__ void score_finish(const ScoreP &p, int64_t row, float
     if (p.status) p.status[row] = uint8_t(stt);
 }
 
-// One workgroup per row, or p.segs of them: workgroup g of a row is then its waves g nw .. of segs nw,
-// and leaves its state for k_score_finish.
-template <int DT, int MK, bool REF, bool KL, bool ENT, bool AL>
+// A row from its records, by one wave: each lane adds records lane, lane + 64, .. in f64, then the lanes'
+// sums in a fixed tree.
+template <int DT, int MK, bool REF, bool KL, bool ENT>
+__device__ __forceinline__ void score_row(const ScoreP &p, int64_t row, const RowRec *rec, int lane) {
+    RowRec r[kScoreRecs / kWave];
+    float af = -INFINITY, arf = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < kScoreRecs / kWave; k++) {
+        r[k] = RowRec{-INFINITY, 0.0f, 0.0f, 0.0f, -INFINITY, 0.0f};
+        if (lane + k * kWave < p.recs) r[k] = rec[lane + k * kWave];
+        af = fmaxf(af, r[k].a);
+        arf = fmaxf(arf, r[k].ar);
+    }
+    af = wave_max3_dpp(af);
+    if constexpr (REF) arf = wave_max3_dpp(arf);
+    RowSums t{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < kScoreRecs / kWave; k++)
+        if (k * kWave < p.recs) rec_add<REF, KL, ENT>(t, r[k], af, arf, p.c);
+    t.S = readlane_d(wave_scan_dpp(t.S), kWave - 1);
+    if constexpr (ENT) t.H = readlane_d(wave_scan_dpp(t.H), kWave - 1);
+    if constexpr (KL) t.B = readlane_d(wave_scan_dpp(t.B), kWave - 1);
+    if constexpr (REF) t.Sr = readlane_d(wave_scan_dpp(t.Sr), kWave - 1);
+    if (lane == 0) score_finish<DT, MK, REF, KL, ENT>(p, row, af, arf, t.S, t.H, t.B, t.Sr);
+}
+
+// A row's chunks go in batches of p.batch consecutive ones, its batches in records of p.per consecutive
+// ones, the records to the waves of the row's p.segs workgroups in turn. Both numbers depend on the
+// vocabulary and the mask's kind alone, and every record is made and merged alike wherever it is made, so
+// a row's bits depend neither on the rows beside it nor on the number of workgroups.
+//
+// A batch is decoded into registers, the wave's next one is loaded, and then its maxima over the wave and
+// its sums relative to them are taken: nothing is rescaled, and the folds over the wave come once per
+// batch. NB = 4 holds 32 values of each input per lane (139 registers with a reference: three waves per
+// SIMD; asking for four spilled, 268 -> 352 us at 8192 x 50304); an f32 mask's words and division take as
+// many again, and there, and for rows of up to 32 chunks, NB = 2. Against a running state per lane over the
+// whole row (us, before / now): 16384 x 8200 bf16 64.2 / 53.0, 300 x 128256 29.7 / 26.4, 8192 x 50304 with a
+// reference 263 / 261, 4096 x 151936 f32 under a u8 mask 453.3 / 450.4.
+template <int DT, int MK, bool REF, bool KL, bool ENT, bool AL, int NB = 4>
 __global__ __launch_bounds__(kScoreThreads) void k_score(ScoreP p) {
-    __shared__ RowState ws[kScoreWaves];
+    __shared__ RowRec ws[kScoreRecs];
     int64_t row = blockIdx.x;
     int seg = 0;
     if (p.segs > 1) {
@@ -213,8 +248,7 @@ __global__ __launch_bounds__(kScoreThreads) void k_score(ScoreP p) {
         seg = int(blockIdx.x % unsigned(p.segs));
     }
     const int lane = threadIdx.x & (kWave - 1);
-    const int wave0 = threadIdx.x / kWave;  // in the workgroup; `wave` of `nw` in the row
-    const int wave = seg * kScoreWaves + wave0;
+    const int wave = __builtin_amdgcn_readfirstlane(seg * kScoreWaves + int(threadIdx.x / kWave));  // in the row
     const int nw = p.segs * kScoreWaves;
     const bool tau_one = p.tau_one != 0;
     const float c = p.c;
@@ -236,190 +270,136 @@ __global__ __launch_bounds__(kScoreThreads) void k_score(ScoreP p) {
                                                                Vb * MaskWords<MK>::kBytes, kBufferWord3)
                            : xres;
 
-    RowState st{-INFINITY, 0.0f, 0.0f, 0.0f, -INFINITY, 0.0f};
-    for (int c0 = wave; c0 < p.nc; c0 += nw * kBatch) {
-        Raw<DT, MK> rx[kBatch];
-        Raw<DT, NT_MASK_NONE> ry[REF ? kBatch : 1];
+    // Chunks c0 .. c0 + p.batch - 1: their maxima over the wave, then their sums relative to them. No
+    // weight exceeds 1, so the sums cannot overflow, and the finishing differences (ln S - ln2 H / S for
+    // the entropy, ln S - ln S_ref for the KL) stay small: no two terms of the size of the logits
+    // cancel. (The maxima pass a NaN by; it stays in the sums.)
+    Raw<DT, MK> rx[NB];
+    Raw<DT, NT_MASK_NONE> ry[REF ? NB : 1];
+    auto load = [&](int c0) {
+        const int n = min(p.batch, p.nc - c0);  // (chunks past it load nothing)
 #pragma unroll
-        for (int b = 0; b < kBatch; b++) {
-            const int ch = c0 + b * nw;
+        for (int b = 0; b < NB; b++) {
+            const int ch = c0 + b;
             if constexpr (AL) {
-                const int e0 = ch < p.nc ? buf_lane_first<DT>(ch, lane) : int(p.V);
+                const int e0 = b < n ? buf_lane_first<DT>(ch, lane) : int(p.V);
                 load_raw_buf<DT, MK>(rx[b], xres, mres, e0);
                 if constexpr (REF) load_raw_buf<DT, NT_MASK_NONE>(ry[b], yres, mres, e0);
             } else {
-                const int64_t e0 = ch < p.nc ? int64_t(ch) * kChunk + lane * kEpl : p.V;
+                const int64_t e0 = b < n ? int64_t(ch) * kChunk + lane * kEpl : p.V;
                 load_raw<DT, MK, AL>(rx[b], xrow, mrow, e0, p.V);
                 if constexpr (REF) load_raw<DT, NT_MASK_NONE, AL>(ry[b], yrow, nullptr, e0, p.V);
             }
         }
+    };
+    auto batch = [&](int c0, int next) -> RowRec {
+        const int n = min(p.batch, p.nc - c0);
+        float v[NB][kEpl], vr[REF ? NB : 1][kEpl];
+        float am = -INFINITY, arm = -INFINITY;
 #pragma unroll
-        for (int b = 0; b < kBatch; b++) {
-            const int ch = c0 + b * nw;
-            if (ch < p.nc) {
-                float v[kEpl], vr[kEpl];
-                decode<DT, MK>(rx[b], v, p.tau, tau_one);
+        for (int b = 0; b < NB; b++) {
+            if (b < n) {
+                decode<DT, MK>(rx[b], v[b], p.tau, tau_one);
                 // The reference logits take the same temperature and vocabulary mask
                 // (reference_kl, rl.rs:347-351).
-                if constexpr (REF) decode_words<DT, MK>(ry[b].x, rx[b].m, vr, p.tau, tau_one);
+                if constexpr (REF) decode_words<DT, MK>(ry[b].x, rx[b].m, vr[b], p.tau, tau_one);
                 if constexpr (AL) {
                     // buffer loads past the row's end read zeros: only the last chunk can hold such
                     // element groups, which take no part in the sums
-                    if (ch == p.nc - 1) {
-                        const int e0 = buf_lane_first<DT>(ch, lane);
+                    if (c0 + b == p.nc - 1) {
+                        const int e0 = buf_lane_first<DT>(c0 + b, lane);
 #pragma unroll
                         for (int j = 0; j < kEpl; j++) {
                             const int e = DT == NT_F32 ? e0 + (j < 4 ? j : kChunk / 2 + j - 4) : e0 + j;
                             if (e >= int(p.V)) {
-                                v[j] = -INFINITY;
-                                vr[j] = -INFINITY;
+                                v[b][j] = -INFINITY;
+                                if constexpr (REF) vr[b][j] = -INFINITY;
                             }
                         }
                     }
                 }
-                // The chunk's weights against the lane's current references. A reference is set
-                // at the first chunk with a finite value and moves (the sums are rescaled and
-                // the chunk weighed again) to the chunk's maximum whenever the lane's 8 weights
-                // of one chunk sum to more than kChunkSumCap: then no weight exceeds kChunkSumCap,
-                // so the reference trails the lane's maximum by at most log2 kChunkSumCap, the
-                // sums cannot overflow, and the finishing differences (ln S - ln2 H / S for the
-                // entropy, ln S - ln S_ref for the KL) stay small: no two terms of the size of the
-                // logits cancel. (A NaN fails the test too, and stays in the sums.)
-                auto rescale = [&](bool pol, bool rf, float an, float anr) {
-                    float dold = 0.0f, eold = 0.0f, f = 1.0f;
-                    if (pol) {
-                        an = fmaxf(an, st.a);
-                        dold = (st.a - shift_of(an)) * c;
-                        f = exp2_hw(dold);
-                        st.a = an;
-                    }
+                const float t = max8_hw(v[b]);
+                am = max3_hw(am, t, t);
+                if constexpr (REF) {
+                    const float tr = max8_hw(vr[b]);
+                    arm = max3_hw(arm, tr, tr);
+                }
+            }
+        }
+        if (next < p.nc) load(next);
+        auto larger = [](float x, float y) { return max3_hw(x, y, y); };
+        if constexpr (REF) {
+            const float both[2] = {am, arm}, m = wave_folds<2>(both, larger);
+            am = readlane_f(m, 0);
+            arm = readlane_f(m, 1);
+        } else {
+            const float one[1] = {am};
+            am = readlane_f(wave_folds<1>(one, larger), 0);
+        }
+        const float sh = shift_of(am), shr = REF ? shift_of(arm) : 0.0f;
+        float S = 0.0f, H = 0.0f, B = 0.0f, Sr = 0.0f;
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            if (b < n) {
+#pragma unroll
+                for (int j = 0; j < kEpl; j++) {
+                    const float d = (v[b][j] - sh) * c;
+                    const float w = exp2_hw(d);
+                    S += w;
+                    if constexpr (ENT) H = fmaf(w, fmaxf(d, -FLT_MAX), H);
                     if constexpr (REF) {
-                        if (rf) {
-                            anr = fmaxf(anr, st.ar);
-                            eold = (st.ar - shift_of(anr)) * c;
-                            st.Sr = exp2_hw(eold) * st.Sr;
-                            st.ar = anr;
-                        }
-                    }
-                    if constexpr (ENT) st.H = f * (st.H + fmaxf(dold, -FLT_MAX) * st.S);
-                    if constexpr (KL) st.B = b_rescaled(st.B, st.S, f, dold, eold);
-                    st.S = f * st.S;
-                };
-                float S, H, Bk, Sr;
-                auto accumulate = [&]() {
-                    const float sh = shift_of(st.a);
-                    float shr = 0.0f;
-                    if constexpr (REF) shr = shift_of(st.ar);
-                    S = st.S, H = st.H, Bk = st.B, Sr = st.Sr;
-#pragma unroll
-                    for (int j = 0; j < kEpl; j++) {
-                        const float d = (v[j] - sh) * c;
-                        const float w = exp2_hw(d);
-                        S += w;
-                        if constexpr (ENT) H = fmaf(w, fmaxf(d, -FLT_MAX), H);
-                        if constexpr (REF) {
-                            const float e = (vr[j] - shr) * c;
-                            Sr += exp2_hw(e);
-                            if constexpr (KL) Bk = fmaf(w, fmaxf(d - e, -FLT_MAX), Bk);
-                        }
-                    }
-                };
-                // A lane's first reference is the maximum of the wave's whole chunk (512 values),
-                // which makes later moves rare. (A wave-uniform branch: every lane takes part in
-                // the DPP maxima.)
-                if (__ballot(st.a == -INFINITY || (REF && st.ar == -INFINITY)) != 0) {
-                    const float wm = wave_max3_dpp(max8_hw(v));
-                    float wmr = -INFINITY;
-                    if constexpr (REF) wmr = wave_max3_dpp(max8_hw(vr));
-                    const bool pol = st.a == -INFINITY, rf = REF && st.ar == -INFINITY;
-                    if (pol || rf) rescale(pol, rf, wm, wmr);
-                }
-                accumulate();
-                {
-                    // the chunk's weight sums (to within rounding, enough for the test)
-                    const bool pol = !(S - st.S <= kChunkSumCap), rf = REF && !(Sr - st.Sr <= kChunkSumCap);
-                    if (pol || rf) {
-                        rescale(pol, rf, max8_hw(v), REF ? max8_hw(vr) : -INFINITY);
-                        accumulate();
+                        const float e = (vr[b][j] - shr) * c;
+                        Sr += exp2_hw(e);
+                        if constexpr (KL) B = fmaf(w, fmaxf(d - e, -FLT_MAX), B);
                     }
                 }
-                st.S = S;
-                if constexpr (ENT) st.H = H;
-                if constexpr (KL) st.B = Bk;
-                if constexpr (REF) st.Sr = Sr;
             }
         }
-    }
-    // Wave tree (lane i takes lane i + o), then the waves in order.
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) {
-        const RowState t = shfl_down_state(st, o);
-        if (lane < o) state_merge<REF, KL, ENT>(st, t, c);
-    }
-    if (lane == 0) ws[wave0] = st;
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    if (p.segs > 1) {
-        st = ws[0];
-        for (int i = 1; i < kScoreWaves; i++) state_merge<REF, KL, ENT>(st, ws[i], c);
-        p.part[blockIdx.x] = st;
-        return;
-    }
+        // the sums asked for, over the lanes: S in lane 0, H, Sr and B in the next ones
+        constexpr int kSums = 1 + ENT + REF + KL, kH = 1, kSr = 1 + ENT, kB = 1 + ENT + REF;
+        float x[kSums > 2 ? 4 : kSums] = {};
+        x[0] = S;
+        if constexpr (ENT) x[kH] = H;
+        if constexpr (REF) x[kSr] = Sr;
+        if constexpr (KL) x[kB] = B;
+        const float t = wave_folds(x, [](float a, float b) { return a + b; });
+        RowRec r{am, readlane_f(t, 0), 0.0f, 0.0f, arm, 0.0f};
+        if constexpr (ENT) r.H = readlane_f(t, kH);
+        if constexpr (REF) r.Sr = readlane_f(t, kSr);
+        if constexpr (KL) r.B = readlane_f(t, kB);
+        return r;
+    };
 
-    // Finish the row in f64.
-    float af = -INFINITY, arf = -INFINITY;
-    for (int i = 0; i < kScoreWaves; i++) {
-        af = fmaxf(af, ws[i].a);
-        arf = fmaxf(arf, ws[i].ar);
-    }
-    double S = 0.0, H = 0.0, B = 0.0, Sr = 0.0;
-    for (int i = 0; i < kScoreWaves; i++) {
-        if (ws[i].S > 0.0f) {
-            const double d = double(ws[i].a - af) * double(c);
-            const double f = exp2(d);
-            S += f * double(ws[i].S);
-            if (ENT) H += f * (double(ws[i].H) + d * double(ws[i].S));
-            if (KL) {
-                const double e = ws[i].ar == -INFINITY ? -INFINITY : double(ws[i].ar - arf) * double(c);
-                B += f * (double(ws[i].B) + (d - e) * double(ws[i].S));
-            }
-        } else if (!(ws[i].S == ws[i].S)) {
-            S = NAN;
+    RowRec *const recs = p.segs > 1 ? p.part + row * p.recs : ws;
+    int c0 = wave < p.recs ? wave * p.per * p.batch : p.nc;
+    if (c0 < p.nc) load(c0);
+    RowRec r;
+    for (int i = wave, k = 0; c0 < p.nc;) {
+        // the batch after this one: the record's next, or the first of the wave's next record
+        int ni = i, nk = k + 1;
+        if (nk == p.per || c0 + p.batch >= p.nc) {
+            ni = i + nw;
+            nk = 0;
         }
-        if (REF && ws[i].ar != -INFINITY) Sr += exp2(double(ws[i].ar - arf) * double(c)) * double(ws[i].Sr);
+        const int next = ni < p.recs ? (ni * p.per + nk) * p.batch : p.nc;
+        const RowRec one = batch(c0, next);
+        if (k == 0) r = one;
+        else rec_merge<REF, KL, ENT>(r, one, c);
+        if (nk == 0 && lane == 0) recs[i] = r;
+        i = ni;
+        k = nk;
+        c0 = next;
     }
-    score_finish<DT, MK, REF, KL, ENT>(p, row, af, arf, S, H, B, Sr);
+    if (p.segs > 1) return;  // (k_score_finish takes them)
+    __syncthreads();
+    if (threadIdx.x < kWave) score_row<DT, MK, REF, KL, ENT>(p, row, ws, lane);
 }
 
-// The rows of a launch with several workgroups per row: a wave per row takes each of its (at most 64)
-// states in one lane, and their sums in index order in f64.
-constexpr int kScoreMaxSegs = kWave;
-
+// The rows of a launch with several workgroups per row, a wave each.
 template <int DT, int MK, bool REF, bool KL, bool ENT>
 __global__ __launch_bounds__(kWave) void k_score_finish(ScoreP p) {
     const int64_t row = blockIdx.x;
-    const int lane = threadIdx.x;
-    RowState s{-INFINITY, 0.0f, 0.0f, 0.0f, -INFINITY, 0.0f};
-    if (lane < p.segs) s = p.part[row * p.segs + lane];
-    const float af = wave_max(s.a), arf = REF ? wave_max(s.ar) : -INFINITY;
-    double S = 0.0, H = 0.0, B = 0.0, Sr = 0.0;
-    if (s.S > 0.0f) {
-        const double d = double(s.a - af) * double(p.c), f = exp2(d);
-        S = f * double(s.S);
-        if (ENT) H = f * (double(s.H) + d * double(s.S));
-        if (KL) {
-            const double e = s.ar == -INFINITY ? -INFINITY : double(s.ar - arf) * double(p.c);
-            B = f * (double(s.B) + (d - e) * double(s.S));
-        }
-    } else if (!(s.S == s.S)) {
-        S = NAN;
-    }
-    if (REF && s.ar != -INFINITY) Sr = exp2(double(s.ar - arf) * double(p.c)) * double(s.Sr);
-    S = readlane_d(wave_scan_dpp(S), kWave - 1);
-    if (ENT) H = readlane_d(wave_scan_dpp(H), kWave - 1);
-    if (KL) B = readlane_d(wave_scan_dpp(B), kWave - 1);
-    if (REF) Sr = readlane_d(wave_scan_dpp(Sr), kWave - 1);
-    if (lane == 0) score_finish<DT, MK, REF, KL, ENT>(p, row, af, arf, S, H, B, Sr);
+    score_row<DT, MK, REF, KL, ENT>(p, row, p.part + row * p.recs, threadIdx.x);
 }
 
 // ------------------------------------------------------------------ fused backward
