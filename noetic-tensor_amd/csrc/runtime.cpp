@@ -54,14 +54,25 @@ int launched(const char *what) {
 // eighth unused); a released one goes on its class's list and is handed out again to work queued
 // later on the library's one stream, the order that hipFreeAsync and hipMallocAsync would give it.
 // At most kKeepTotal bytes are kept: past it the blocks go back to the device's pool, and so do
-// all of them when the pool has no memory left. Calls made under capture take their memory from
-// the pool, as graph nodes. All of it under the context's lock.
+// all of them when the pool has no memory left. All of it under the context's lock.
+// While the stream is captured, calls take their memory from the pool, as graph nodes, and no kept
+// block goes back to it (the free would become a node of the caller's graph, and run at each
+// replay). A block released during a capture may be one that the graph's replays work on, so
+// it stays allocated for good and is handed out to nobody; one released before goes on its list.
 constexpr size_t kKeepBlock = size_t(128) << 20, kKeepTotal = size_t(512) << 20;
 constexpr int kKeepClasses = 8 * 28;
 struct KeptBlock {
     int cls;
     bool used;
 };
+
+// Whether the library stream is being captured.
+static int capturing(bool *out) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (int rc = hip_check(hipStreamIsCapturing(ctx().stream, &cap), "hipStreamIsCapturing")) return rc;
+    *out = cap != hipStreamCaptureStatusNone;
+    return 0;
+}
 struct Kept {
     std::unordered_map<void *, KeptBlock> blocks;
     std::vector<void *> lists[kKeepClasses];
@@ -110,22 +121,20 @@ static int take_block(size_t bytes, void **out) {
     Kept &k = kept();
     size_t size = bytes;
     int cls = -1;
-    if (bytes <= kKeepBlock) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (int rc = hip_check(hipStreamIsCapturing(c.stream, &cap), "hipStreamIsCapturing")) return rc;
-        if (cap == hipStreamCaptureStatusNone) {
-            cls = size_class(bytes, &size);
-            if (!k.lists[cls].empty()) {
-                *out = k.lists[cls].back();
-                k.lists[cls].pop_back();
-                k.bytes -= size;
-                k.blocks[*out].used = true;
-                return 0;
-            }
+    bool cap = false;
+    if (int rc = capturing(&cap)) return rc;
+    if (bytes <= kKeepBlock && !cap) {
+        cls = size_class(bytes, &size);
+        if (!k.lists[cls].empty()) {
+            *out = k.lists[cls].back();
+            k.lists[cls].pop_back();
+            k.bytes -= size;
+            k.blocks[*out].used = true;
+            return 0;
         }
     }
     hipError_t e = hipMallocAsync(out, size, c.stream);
-    if (e == hipErrorOutOfMemory && k.bytes > 0) {
+    if (e == hipErrorOutOfMemory && k.bytes > 0 && !cap) {
         (void)hipGetLastError();
         if (int rc = drop_kept(0)) return rc;
         e = hipMallocAsync(out, size, c.stream);
@@ -135,25 +144,34 @@ static int take_block(size_t bytes, void **out) {
     return 0;
 }
 
-static int give_block(void *p) {
+// `in_capture`: the release was made while the stream was captured.
+static int give_block(void *p, bool in_capture) {
     Kept &k = kept();
     auto it = k.blocks.find(p);
     if (it == k.blocks.end()) return hip_check(hipFreeAsync(p, ctx().stream), "hipFreeAsync");
     if (!it->second.used) return hip_check(hipErrorInvalidValue, "free of a block that is not in use");
     it->second.used = false;
+    if (in_capture) return 0;
     k.lists[it->second.cls].push_back(p);
     k.bytes += class_bytes(it->second.cls);
+    if (k.bytes <= kKeepTotal) return 0;
+    bool cap = false;
+    if (int rc = capturing(&cap)) return rc;
+    if (cap) return 0;  // (a later release trims them)
     // the larger blocks first: from 1 MiB (class 8 * 20) up, then all
-    if (k.bytes > kKeepTotal)
-        if (int rc = drop_kept(8 * 20)) return rc;
+    if (int rc = drop_kept(8 * 20)) return rc;
     return k.bytes > kKeepTotal ? drop_kept(0) : 0;
 }
 
 // Pointers released by nt_hip_free since the last entry, freed on the stream by the next one
 // (the reference's PENDING_FREE, src/tensor/cuda/backend.rs:35-45 and 222-243: a release only
 // records the pointer, so it never waits for the device or for the context's lock).
+struct Pending {
+    void *ptr;
+    bool in_capture;
+};
 static std::mutex g_pending_mu;
-static std::vector<void *> g_pending;
+static std::vector<Pending> g_pending;
 
 int enter_nofree(std::unique_lock<std::mutex> *out) {
     Ctx &c = ctx();
@@ -171,20 +189,20 @@ int enter(std::unique_lock<std::mutex> *out) {
     if (c.device < 0) return fail(NT_E_UNCLAIMED, "no HIP device claimed in this process (nt_hip_claim)");
     hipError_t e = hipSetDevice(c.device);
     if (e != hipSuccess) return hip_check(e, "hipSetDevice");
-    std::vector<void *> freed;
+    std::vector<Pending> freed;
     {
         std::lock_guard<std::mutex> pl(g_pending_mu);
         freed.swap(g_pending);
     }
     for (size_t i = 0; i < freed.size(); ++i) {
         // the work queued before the release still runs first: the free is ordered after it
-        void *p = freed[i];
+        const Pending p = freed[i];
         int rc = 0;
         if (c.pools) {
-            rc = give_block(p);
+            rc = give_block(p.ptr, p.in_capture);
         } else {
             rc = hip_check(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
-            if (!rc) rc = hip_check(hipFree(p), "hipFree");
+            if (!rc) rc = hip_check(hipFree(p.ptr), "hipFree");
         }
         if (rc) {
             // keep what is not freed yet for the next entry
@@ -206,9 +224,9 @@ int scratch_alloc(size_t bytes, void **out) {
 
 int scratch_release(void *ptr) {
     if (!ptr) return 0;
-    if (ctx().pools) return give_block(ptr);
+    if (ctx().pools) return give_block(ptr, false);  // (taken by the same call: kept, or a graph node's)
     std::lock_guard<std::mutex> pl(g_pending_mu);
-    g_pending.push_back(ptr);
+    g_pending.push_back(Pending{ptr, false});
     return 0;
 }
 
@@ -350,8 +368,10 @@ int nt_hip_alloc(size_t bytes, void **out) {
 
 int nt_hip_free(void *ptr) {
     if (!ptr) return 0;
+    bool cap = false;
+    if (ctx().stream && capturing(&cap)) cap = true;  // (not known: as if it were)
     std::lock_guard<std::mutex> pl(g_pending_mu);
-    g_pending.push_back(ptr);
+    g_pending.push_back(Pending{ptr, cap});
     return 0;
 }
 
