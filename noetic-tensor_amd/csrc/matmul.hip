@@ -508,6 +508,25 @@ __global__ __launch_bounds__(256) void k_half_tiles(MatmulP p, const uint8_t *pa
 
 template <bool HALF, class C, bool SPLIT>
 int launch_matmul(const MatmulP &p, hipStream_t s) {
+    // A launch holds fewer than 2^32 threads. More blocks, as of millions of small batches, go in halves
+    // along the outermost batch dimension that has any.
+    if (p.blocks > ((int64_t(1) << 32) - 1) / C::kThreads) {
+        int d = 0;
+        while (d < p.nbd && p.bshape[d] == 1) d++;
+        if (d == p.nbd) return fail(NT_E_ARG, "matmul: too many output tiles");
+        int64_t inner = int64_t(p.m) * p.n, tiles = int64_t(p.tm) * p.tn;
+        for (int e = d + 1; e < p.nbd; e++) inner *= p.bshape[e], tiles *= p.bshape[e];
+        MatmulP q = p;
+        q.bshape[d] = p.bshape[d] / 2;
+        q.blocks = q.bshape[d] * tiles;
+        if (int rc = launch_matmul<HALF, C, SPLIT>(q, s)) return rc;
+        q.a_off += q.bshape[d] * p.a_bs[d];
+        q.b_off += q.bshape[d] * p.b_bs[d];
+        q.c += q.bshape[d] * inner;
+        q.bshape[d] = p.bshape[d] - q.bshape[d];
+        q.blocks = q.bshape[d] * tiles;
+        return launch_matmul<HALF, C, SPLIT>(q, s);
+    }
     const dim3 grid(unsigned(p.blocks)), block(C::kThreads);
     const bool ak = p.a_cs == 1, bn = p.b_cs == 1 || p.b_rs != 1;
     if (ak && bn) hipLaunchKernelGGL((k_matmul<HALF, C, true, true, SPLIT>), grid, block, 0, s, p);

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import noetic_rl as nr
-from noetic_ops import DTensor
+from noetic_ops import DTensor, MatmulPrecision
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -85,3 +85,27 @@ def test_tiles_and_splits(m, k, n, ta, tb):
     rng = np.random.default_rng(m + k)
     a, b = values("wide", (m, k), rng, True), values("wide", (k, n), rng, False)
     assert same(product(a, b, ta, tb), O.matmul(a, b))
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 300, 64), (64, 16, 1), (65, 40, 65), (128, 24, 64), (100, 32, 40), (3, 8, 5)])
+@pytest.mark.parametrize("half", [False, True])
+def test_many_small_batches(m, k, n, half):
+    """Batches enough for 128 tiles, with sides that 64 tiles cover with less; a last panel of whole groups."""
+    rng = np.random.default_rng(m + k)
+    a, b = (rng.integers(-9, 10, (300,) + s).astype(F) for s in ((m, k), (k, n)))
+    if not half:
+        a *= F(1.1)
+    got = DTensor.from_numpy(a).matmul_with(DTensor.from_numpy(b), MatmulPrecision.HALF if half else MatmulPrecision.F32)
+    got = got.to_numpy()
+    for z in (0, 1, 150, 299):
+        assert same(got[z], a[z] @ b[z] if half else O.matmul(a[z], b[z])), z
+
+
+@pytest.mark.parametrize("half", [False, True])
+def test_more_batches_than_one_launch_holds(half):
+    """17 million workgroups of 256 threads: over the 2^32 threads of a launch."""
+    nb = 17_000_003
+    a = DTensor.from_numpy((np.arange(nb) % 251).astype(F).reshape(nb, 1, 1))
+    b = DTensor.from_numpy(np.full((1, 1, 1), 3, F))
+    got = a.matmul_with(b, MatmulPrecision.HALF if half else MatmulPrecision.F32).to_numpy().ravel()
+    np.testing.assert_array_equal(got, 3 * (np.arange(nb) % 251).astype(F))
