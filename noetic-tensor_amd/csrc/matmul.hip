@@ -93,9 +93,14 @@ __device__ __forceinline__ void load8(const float *src, int64_t stride, f32x4_t 
 }
 
 // The same of the last panel, when K does not end with it: elements at or past `lim` are `pad`.
+template <bool K1>
 __device__ __forceinline__ void load8_tail(const float *src, int64_t stride, int lim, float pad, f32x4_t (&x)[2]) {
+    if (lim >= 8) {
+        load8<K1>(src, stride, x);
+    } else {
 #pragma unroll
-    for (int e = 0; e < 8; e++) x[e / 4][e % 4] = e < lim ? src[e * stride] : pad;
+        for (int e = 0; e < 8; e++) x[e / 4][e % 4] = e < lim ? src[e * stride] : pad;
+    }
 }
 
 // A tile of NM x NN waves, each WM x WN MFMA tiles of 32 x 32. Two waves per SIMD (eight per 128 x 128
@@ -326,17 +331,19 @@ __global__ __launch_bounds__(C::kThreads, 2) void k_matmul(MatmulP p) {
     if (kfull < kend) {  // the last panel, when K ends inside it
 #pragma unroll
         for (int q = 0; q < GA; q++)
-            load8_tail(asrc[q] + int64_t(kfull) * p.a_cs, p.a_cs, K - kfull - akg[q], kPadA, ra[0][q]);
+            load8_tail<AK>(asrc[q] + int64_t(kfull) * p.a_cs, p.a_cs, K - kfull - akg[q], kPadA, ra[0][q]);
 #pragma unroll
         for (int q = 0; q < GB; q++)
-            load8_tail(bsrc[q] + int64_t(kfull) * p.b_rs, p.b_rs, K - kfull - bkg[q], 0.0f, rb[0][q]);
-        __syncthreads();  // (the reads of the last whole panel are done)
+            load8_tail<!BN>(bsrc[q] + int64_t(kfull) * p.b_rs, p.b_rs, K - kfull - bkg[q], 0.0f, rb[0][q]);
+        if (kbeg < kfull) __syncthreads();  // (the reads of the last whole panel are done)
         stash(0, ra[0], rb[0]);
         __syncthreads();
 #pragma unroll
         for (int kg = 0; kg < 4; kg++) {
-            fetch(0, kg);
-            group(kg);
+            if (kfull + kg * (kBK / 4) < kend) {  // (a quarter past k's end holds padding alone)
+                fetch(0, kg);
+                group(kg);
+            }
         }
         close(kfull);
     }
@@ -536,6 +543,16 @@ int launch_matmul(const MatmulP &p, hipStream_t s) {
     return launched(HALF ? "k_matmul (half)" : "k_matmul");
 }
 
+// 128 x 128 tiles when they give at least `least` workgroups, else 64 x 64; also 64 x 64 where these cover
+// the outputs with half the area (a side of at most 64, as of many small batches). Measured (us, 128 / 64):
+// 256 batches of 1 x 4096 x 64 291 / 91, 20000 of 4 x 4 x 4 269 / 81, 300 of 100 x 40 x 30 15.3 / 9.5; half, 4096
+// of 16 x 16 x 16 34.2 / 17.8, 64 x 256 x 50304 30.7 / 30.9.
+int tile_side(int64_t batches, int64_t m, int64_t n, int64_t least) {
+    const int64_t big = batches * ((m + 127) / 128) * ((n + 127) / 128);
+    const int64_t small = batches * ((m + 63) / 64) * ((n + 63) / 64);
+    return big >= least && small > 2 * big ? 128 : 64;
+}
+
 template <bool HALF, bool SPLIT>
 int launch_tile(int tile, const MatmulP &p, hipStream_t s) {
     if (tile == 128) return launch_matmul<HALF, Tile128, SPLIT>(p, s);
@@ -592,8 +609,7 @@ int nt_hip_matmul(const float *a, const NtLayout *al, const float *b, const NtLa
     // 128x128 tiles when they give every CU of the 256 a workgroup, else 64x64. Measured (us, 128 /
     // 64 tiles): 2048^3 (256 tiles of 128) 142 / 161, 1500 x 700 x 1900 (180) 54.3 / 46.9, 1024^3 (64)
     // 72.7 / 27.7.
-    const int64_t big = nb * ((m + 127) / 128) * ((n + 127) / 128);
-    const int T = big >= 256 ? 128 : 64;
+    const int T = tile_side(nb, m, n, 256);
     p.tm = int32_t((m + T - 1) / T);
     p.tn = int32_t((n + T - 1) / T);
     const int64_t tiles = nb * p.tm * p.tn;
@@ -713,8 +729,7 @@ int nt_hip_matmul_half(const float *a, const NtLayout *al, const float *b, const
     }
     // 128 x 128 tiles from 160 of them on, else 64 x 64. Measured (us, 128 / 64): 1500 x 700 x 1900 (180
     // tiles of 128) 19.5 / 25.2; 4096 x 4096 x 512 (128) 56.7 / 51.2.
-    const int64_t big = nb * ((m + 127) / 128) * ((n + 127) / 128);
-    const int T = big >= 160 ? 128 : 64;
+    const int T = tile_side(nb, m, n, 160);
     p.tm = int32_t((m + T - 1) / T);
     p.tn = int32_t((n + T - 1) / T);
     p.blocks = nb * p.tm * p.tn;
