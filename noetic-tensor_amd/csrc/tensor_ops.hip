@@ -10,6 +10,7 @@
 // instantiated per merged rank, so the coordinate loop unrolls.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <string>
@@ -397,40 +398,46 @@ __global__ __launch_bounds__(kOpsThreads) void k_binary(int op, const float *__r
 // no index is divided, and with V = 4 (16-byte aligned rows, C % 4 == 0) every access is 16 bytes.
 // Bound by HBM. [256, 50304] less a value per row: 26.9 -> 16.1 us (6.4 TB/s) over the element loop.
 constexpr int kRowsPer = 4;  // groups of 256 V columns per workgroup
-template <int OP, int V, int AM, int BM>
+template <int OP, int V, int AM, int BM, bool MORE>
 __global__ __launch_bounds__(kOpsThreads) void k_binary_rows(const float *__restrict__ a, int64_t ars,
                                                              const float *__restrict__ b, int64_t brs,
                                                              float *__restrict__ y, int64_t rows, int64_t C) {
     typedef float vec __attribute__((ext_vector_type(V)));
-    const int64_t c0 = int64_t(blockIdx.x) * (kRowsPer * kOpsThreads * V) + threadIdx.x * V;
+    constexpr int64_t kPer = kRowsPer * kOpsThreads * V;
     for (int64_t row = blockIdx.y; row < rows; row += gridDim.y) {
         const float *ar = a + row * ars, *br = b + row * brs;
         const float as = AM ? 0.0f : ar[0], bs = BM ? 0.0f : br[0];
-        vec p[kRowsPer], q[kRowsPer];
+        auto columns = [&](int64_t c0) {
+            vec p[kRowsPer], q[kRowsPer];
 #pragma unroll
-        for (int u = 0; u < kRowsPer; u++) {
-            const int64_t c = c0 + u * (kOpsThreads * V);
-            p[u] = vec(as);
-            q[u] = vec(bs);
-            if (c < C) {
-                if (AM) p[u] = *reinterpret_cast<const vec *>(ar + c);
-                if (BM) q[u] = *reinterpret_cast<const vec *>(br + c);
+            for (int u = 0; u < kRowsPer; u++) {
+                const int64_t c = c0 + u * (kOpsThreads * V);
+                p[u] = vec(as);
+                q[u] = vec(bs);
+                if (c < C) {
+                    if (AM) p[u] = *reinterpret_cast<const vec *>(ar + c);
+                    if (BM) q[u] = *reinterpret_cast<const vec *>(br + c);
+                }
             }
-        }
 #pragma unroll
-        for (int u = 0; u < kRowsPer; u++) {
-            const int64_t c = c0 + u * (kOpsThreads * V);
-            if (c >= C) continue;
-            vec r;
+            for (int u = 0; u < kRowsPer; u++) {
+                const int64_t c = c0 + u * (kOpsThreads * V);
+                if (c >= C) continue;
+                vec r;
 #pragma unroll
-            for (int e = 0; e < V; e++) {
-                if constexpr (OP == NT_BIN_ADD) r[e] = p[u][e] + q[u][e];
-                else if constexpr (OP == NT_BIN_SUB) r[e] = p[u][e] - q[u][e];
-                else if constexpr (OP == NT_BIN_MUL) r[e] = p[u][e] * q[u][e];
-                else r[e] = div_f(p[u][e], q[u][e]);
+                for (int e = 0; e < V; e++) {
+                    if constexpr (OP == NT_BIN_ADD) r[e] = p[u][e] + q[u][e];
+                    else if constexpr (OP == NT_BIN_SUB) r[e] = p[u][e] - q[u][e];
+                    else if constexpr (OP == NT_BIN_MUL) r[e] = p[u][e] * q[u][e];
+                    else r[e] = div_f(p[u][e], q[u][e]);
+                }
+                *reinterpret_cast<vec *>(y + row * C + c) = r;
             }
-            *reinterpret_cast<vec *>(y + row * C + c) = r;
-        }
+        };
+        int64_t c0 = int64_t(blockIdx.x) * kPer + threadIdx.x * V;
+        columns(c0);
+        if constexpr (MORE)
+            for (c0 += int64_t(gridDim.x) * kPer; c0 < C; c0 += int64_t(gridDim.x) * kPer) columns(c0);
     }
 }
 
@@ -444,17 +451,23 @@ bool launch_binary_rows(int op, const float *a, const View &av, const float *b, 
     const int64_t ars = R == 2 ? av.st[0] : 0, brs = R == 2 ? bv.st[0] : 0;
     a += av.off;
     b += bv.off;
-    auto whole = [](const float *x, int64_t m, int64_t rs) {
+    auto aligned = [](const float *x, int64_t m, int64_t rs) {
         return m == 0 || (reinterpret_cast<uintptr_t>(x) % 16 == 0 && rs % 4 == 0);
     };
-    const bool v4 = C % 4 == 0 && whole(a, am, ars) && whole(b, bm, brs) && reinterpret_cast<uintptr_t>(y) % 16 == 0;
-    const int64_t per = int64_t(kRowsPer) * kOpsThreads * (v4 ? 4 : 1), bx = (C + per - 1) / per;
-    if (bx > 0x7fffffff) return false;
+    const bool v4 = C % 4 == 0 && aligned(a, am, ars) && aligned(b, bm, brs) && reinterpret_cast<uintptr_t>(y) % 16 == 0;
+    const int64_t per = int64_t(kRowsPer) * kOpsThreads * (v4 ? 4 : 1);
+    const int64_t whole = (C + per - 1) / per;
+    int64_t bx = std::min<int64_t>(whole, 1 << 20);  // (a launch holds fewer than 2^32 threads)
+    // One row against all (its reads hit the caches), many rows of little over one workgroup's columns: a
+    // second one for a few columns costs what a full one does, and is left to the first's second turn
+    // (40000 x 4100 386 -> 248 us, 363 by the element loop; the other forms lose by it).
+    if (bx == 2 && C - per < per / 8 && rows >= 2048 && am && bm && (ars == 0 || brs == 0)) bx = 1;
     const dim3 grid(unsigned(bx), unsigned(rows < 32768 ? rows : 32768));
-    auto go = [&](auto opc) {
+    auto go = [&](auto opc, auto morec) {
         constexpr int OP = decltype(opc)::value;
-#define NT_ROWS(V, AM, BM) \
-    hipLaunchKernelGGL((k_binary_rows<OP, V, AM, BM>), grid, dim3(kOpsThreads), 0, s, a, ars, b, brs, y, rows, C)
+        constexpr bool MORE = decltype(morec)::value;
+#define NT_ROWS(V, AM, BM)                                                                                         \
+    hipLaunchKernelGGL((k_binary_rows<OP, V, AM, BM, MORE>), grid, dim3(kOpsThreads), 0, s, a, ars, b, brs, y, rows, C)
         if (v4) {
             if (am && bm) NT_ROWS(4, 1, 1);
             else if (am) NT_ROWS(4, 1, 0);
@@ -466,10 +479,14 @@ bool launch_binary_rows(int op, const float *a, const View &av, const float *b, 
         }
 #undef NT_ROWS
     };
-    if (op == NT_BIN_ADD) go(std::integral_constant<int, NT_BIN_ADD>{});
-    else if (op == NT_BIN_SUB) go(std::integral_constant<int, NT_BIN_SUB>{});
-    else if (op == NT_BIN_MUL) go(std::integral_constant<int, NT_BIN_MUL>{});
-    else go(std::integral_constant<int, NT_BIN_DIV>{});
+    auto by_more = [&](auto opc) {
+        if (bx < whole) go(opc, std::true_type{});
+        else go(opc, std::false_type{});
+    };
+    if (op == NT_BIN_ADD) by_more(std::integral_constant<int, NT_BIN_ADD>{});
+    else if (op == NT_BIN_SUB) by_more(std::integral_constant<int, NT_BIN_SUB>{});
+    else if (op == NT_BIN_MUL) by_more(std::integral_constant<int, NT_BIN_MUL>{});
+    else by_more(std::integral_constant<int, NT_BIN_DIV>{});
     return true;
 }
 

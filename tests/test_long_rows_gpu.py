@@ -95,3 +95,27 @@ def test_binary_over_rows(op, rows, cols, off):
                          (full, one, X, y[:1, :1]), (one, full, x[:1, :1], Y), (row, full, X[:1], Y), (col, row, X[:, :1], Y[:1])]:
         got = ops.binary(op, a, al, b, bl).to_numpy()
         np.testing.assert_array_equal(got.view(np.uint32), np.broadcast_to(f(u, v), X.shape).astype(F).view(np.uint32))
+
+
+# both sides of each line between the two kernels, and last tiles that end at, before and past a group of 32
+# values per chain
+@pytest.mark.parametrize("rows,n", [(3, 4999), (3, 5000), (64, 4095), (64, 4096), (64, 4104), (64, 4344), (64, 4352), (64, 4361),
+                                    (513, 8191), (520, 8200), (769, 16383), (1024, 16390), (1025, 16384)])
+def test_sum_where_the_kernels_change(rows, n):
+    rng = np.random.default_rng(rows + n)
+    x = (rng.standard_normal((rows, n)) * np.exp(rng.standard_normal((rows, n)) * 3)).astype(F)
+    x[0] = -0.0
+    x[1, -1] = np.inf
+    got = ops.reduce_dim(ReduceOp.SUM, nr.Tensor.from_numpy(x), (rows, n), 1).to_numpy().ravel()
+    for r in [0, 1, 2, rows // 2, rows - 1]:
+        assert got[r].view(np.uint32) == cpuref_sum(x[r]).view(np.uint32), r
+
+
+@pytest.mark.parametrize("rows,cols", [(2048, 1030), (2049, 4100), (2047, 4100), (3, 4100), (2100, 1160)])
+def test_one_row_against_many_of_little_over_a_workgroup(rows, cols):
+    rng = np.random.default_rng(cols)
+    x, y = rng.standard_normal((rows, cols)).astype(F), rng.standard_normal(cols).astype(F)
+    a, b = nr.Tensor.from_numpy(x), nr.Tensor.from_numpy(y)
+    full, row = Layout([rows, cols], [cols, 1], 0), Layout([rows, cols], [0, 1], 0)
+    np.testing.assert_array_equal(ops.binary(BinaryOp.SUB, a, full, b, row).to_numpy(), x - y)
+    np.testing.assert_array_equal(ops.binary(BinaryOp.SUB, b, row, a, full).to_numpy(), y - x)
