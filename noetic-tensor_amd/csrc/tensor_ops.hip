@@ -547,7 +547,8 @@ __global__ __launch_bounds__(kOpsThreads) void k_sum_last(const float *__restric
 // whose lanes read their chains from memory. (Reading 32 values ahead of the adds took 40.7.)
 constexpr int kSumTile = 4096, kSumChain = kSumTile / 8, kSumStride = kSumChain + 8;
 constexpr int kSumLoaders = 256, kSumPer = kSumTile / kSumLoaders;
-__global__ __launch_bounds__(kSumLoaders + kWave) void k_sum_long(const float *__restrict__ x, int64_t outer, int64_t n,
+// (four waves per SIMD asked for: two workgroups of five fit a CU)
+__global__ __launch_bounds__(kSumLoaders + kWave, 4) void k_sum_long(const float *__restrict__ x, int64_t outer, int64_t n,
                                                                   float *__restrict__ y) {
     __shared__ __attribute__((aligned(16))) float s[2][8 * kSumStride];
     const bool adds = threadIdx.x < kWave;
@@ -570,23 +571,21 @@ __global__ __launch_bounds__(kSumLoaders + kWave) void k_sum_long(const float *_
         float p = 0.0f;
         auto add = [&](int64_t t, int b) {
             const float *c = &s[b][g * kSumStride];
-            if ((t + 1) * kSumTile <= n8) {
+            // (a last tile's values past the row are zeros, and p, begun at +0, is never -0: adding
+            // them leaves it as it is)
+            const int m = int(min(int64_t(kSumChain), n8 / 8 - t * kSumChain));
 #pragma unroll 1
-                for (int q = 0; q < kSumChain; q += 32) {
-                    float4 w[8];
+            for (int q = 0; q < m; q += 32) {
+                float4 w[8];
 #pragma unroll
-                    for (int i = 0; i < 8; i++) w[i] = *reinterpret_cast<const float4 *>(c + q + 4 * i);
+                for (int i = 0; i < 8; i++) w[i] = *reinterpret_cast<const float4 *>(c + q + 4 * i);
 #pragma unroll
-                    for (int i = 0; i < 8; i++) {
-                        p = p + w[i].x;
-                        p = p + w[i].y;
-                        p = p + w[i].z;
-                        p = p + w[i].w;
-                    }
+                for (int i = 0; i < 8; i++) {
+                    p = p + w[i].x;
+                    p = p + w[i].y;
+                    p = p + w[i].z;
+                    p = p + w[i].w;
                 }
-            } else {
-                const int m = int(n8 - t * kSumTile) / 8;
-                for (int q = 0; q < m; q++) p = p + c[q];
             }
         };
         if (!adds) {
@@ -630,10 +629,12 @@ __global__ __launch_bounds__(kSumLoaders + kWave) void k_sum_long(const float *_
 }
 
 int launch_sum_last(const float *x, int64_t outer, int64_t n, float *y, hipStream_t s) {
-    // A row per workgroup pays where rows are long and too few for their chains to fill the chip.
-    // Measured (us, k_sum_long / k_sum_last): 8 x 50304 31 / 41, 256 x 50304 31 / 115, 2048 x 50304
-    // 161 / 178, 1 x 4000000 1709 / 3990; 16384 x 4096 234 / 54, 4096 x 2048 131 / 6.5, 256 x 2048 13.5 / 5.9.
-    if ((n >= 4096 && outer <= 512) || (n >= 16384 && outer <= 2048)) {
+    // A row per workgroup pays where rows are long and too few for their chains to fill the chip; three
+    // such workgroups fit a CU. Measured (us, k_sum_long / k_sum_last): 1 x 4096 6.2 / 4.8, 8 x 6000 7.0 /
+    // 9.2, 512 x 4096 7.7 / 9.1, 700 x 4096 12.1 / 9.1, 700 x 8192 14.5 / 16.8, 1024 x 12000 30.6 / 31.3, 1024
+    // x 8192 23.3 / 17.2, 2048 x 50304 145 / 177, 2048 x 32768 95 / 76; 256 x 50304 27 / 114.
+    const int64_t least = outer <= 32 ? 5000 : outer <= 512 ? 4096 : outer <= 768 ? 8192 : outer <= 1024 ? 16384 : 50000;
+    if (outer <= 2048 && n >= least) {
         hipLaunchKernelGGL(k_sum_long, dim3(unsigned(outer < kMaxBlocks ? outer : kMaxBlocks)), dim3(kSumLoaders + kWave),
                            0, s, x, outer, n, y);
     } else {
