@@ -685,6 +685,9 @@ __device__ __forceinline__ Best shfl_best(Best b, int src_lane_delta) {
 // One 1024-thread block per lane of the last axis (or per lane of everything, outer = 1): each
 // thread picks over its strided subsequence, then the block combines.
 constexpr int kBestThreads = 1024;
+// DEEP (rows of 8192 or more): eight loads in flight; one at a time leaves the row's read bound by its
+// latency, [256, 50304] 21.6 -> 12.1 us.
+template <bool DEEP>
 __global__ __launch_bounds__(kBestThreads) void k_best_last(const float *__restrict__ x, int64_t outer, int64_t n,
                                                             float *__restrict__ val, int32_t *__restrict__ idx) {
     __shared__ Best wb[kBestThreads / kWave];
@@ -704,18 +707,18 @@ __global__ __launch_bounds__(kBestThreads) void k_best_last(const float *__restr
                     bk = k;
                 }
             };
-            // (eight loads in flight: one at a time left the row's read bound by its latency, [256,
-            // 50304] 21.6 -> 12.1 us)
-            constexpr int kB = 8;
             int64_t k = threadIdx.x;
-            for (; k + (kB - 1) * kBestThreads < n; k += kB * kBestThreads) {
-                float e[kB];
+            if constexpr (DEEP) {
+                constexpr int kB = 8;
+                for (; k + (kB - 1) * kBestThreads < n; k += kB * kBestThreads) {
+                    float e[kB];
 #pragma unroll
-                for (int i = 0; i < kB; i++) e[i] = r[k + i * kBestThreads];
+                    for (int i = 0; i < kB; i++) e[i] = r[k + i * kBestThreads];
 #pragma unroll
-                for (int i = 0; i < kB; i++) take(e[i], int32_t(k + i * kBestThreads));
+                    for (int i = 0; i < kB; i++) take(e[i], int32_t(k + i * kBestThreads));
+                }
             }
-            for (; k < n; k += kBestThreads) take(r[k], int32_t(k));
+            for (int32_t j = int32_t(k); j < int32_t(n); j += kBestThreads) take(r[j], j);
             b = Best{bv, bk};
         } else {
             for (int64_t k = threadIdx.x; k < n; k += kBestThreads) b = pick(b, Best{r[k], k});
@@ -734,6 +737,12 @@ __global__ __launch_bounds__(kBestThreads) void k_best_last(const float *__restr
         }
         __syncthreads();
     }
+}
+
+void launch_best_last(const float *x, int64_t outer, int64_t n, float *val, int32_t *idx, hipStream_t s) {
+    const dim3 grid(unsigned(outer < kMaxBlocks ? outer : kMaxBlocks)), block(kBestThreads);
+    if (n >= 8 * kBestThreads) hipLaunchKernelGGL(k_best_last<true>, grid, block, 0, s, x, outer, n, val, idx);
+    else hipLaunchKernelGGL(k_best_last<false>, grid, block, 0, s, x, outer, n, val, idx);
 }
 
 // The same pick of short rows, a wave per row: no barrier, and no 1024-thread combine that a row of a few
@@ -1014,8 +1023,7 @@ int nt_hip_reduce_dim(int32_t op, const float *x, int64_t outer, int64_t n, int6
                                outer, int32_t(n), val, idx);
             return launched("reduce_dim max");
         }
-        const int64_t b = outer > kMaxBlocks ? kMaxBlocks : outer;
-        hipLaunchKernelGGL(k_best_last, dim3(unsigned(b)), dim3(kBestThreads), 0, s, x, outer, n, val, idx);
+        launch_best_last(x, outer, n, val, idx, s);
     } else {
         hipLaunchKernelGGL(k_best_mid, dim3(blocks_for(lanes)), dim3(kOpsThreads), 0, s, x, outer, n, inner, val, idx);
     }
@@ -1032,7 +1040,7 @@ int nt_hip_reduce_all(int32_t op, const float *x, int64_t n, float *out) {
     if (int rc = enter(&lk)) return rc;
     hipStream_t s = ctx().stream;
     if (op == NT_RED_SUM) return launch_sum_last(x, 1, n, out, s);
-    hipLaunchKernelGGL(k_best_last, dim3(1), dim3(kBestThreads), 0, s, x, int64_t(1), n, out, (int32_t *)nullptr);
+    launch_best_last(x, 1, n, out, nullptr, s);
     return launched("reduce_all");
 }
 
