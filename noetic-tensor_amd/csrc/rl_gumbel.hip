@@ -53,8 +53,8 @@ void launch_gumbel(const GumbelP &p, int64_t rows, int threads, hipStream_t s) {
                 gumbel_queue_bytes(threads, GREEDY, DT, MK), s, p);
     if (p.segs > 1) {
         std::snprintf(nm, sizeof nm, "nt::k_gumbel_finish<%d, %d, %s, %s>", DT, MK, rtc_bool(ODD), rtc_bool(GREEDY));
-        launch_path(k_gumbel_finish<DT, MK, ODD, GREEDY>, nm, dim3(unsigned(rows)), dim3(kGumbelMaxThreads),
-                    gumbel_queue_bytes(kGumbelMaxThreads, GREEDY, DT, MK), s, p);
+        launch_path(k_gumbel_finish<DT, MK, ODD, GREEDY>, nm, dim3(unsigned(rows)),
+                    dim3(GREEDY ? 64 : kGumbelMaxThreads), gumbel_queue_bytes(kGumbelMaxThreads, GREEDY, DT, MK), s, p);
     }
 }
 
@@ -78,9 +78,13 @@ int gumbel_recs(GumbelRec **out) {
 // Workgroups per row: about one per CU, each of at least 128 blocks (more pay their start, their partial
 // last step and their reductions again). Measured (us, one workgroup per row / this rule): 1 row of
 // 32000 f32 44.9 / 9.8, 16 of 50304 bf16 66.3 / 12.3, 64 of 32001 f32 48.9 / 18.6, 128 of 128256 bf16
-// under a shared f32 mask 81.7 / 51.8; with twice the workgroups 9.8, 12.5, 17.3 and 62.0.
-int gumbel_segs(int64_t rows, int64_t nblk) {
-    const int64_t g = std::min<int64_t>(256 / rows, nblk / 128);
+// under a shared f32 mask 81.7 / 51.8; with twice the workgroups 9.8, 12.5, 17.3 and 62.0. Under 400 blocks
+// the second launch costs more than it saves (64 rows of 2049 f32 under a u8 mask 14.6 / 17.5, 1 of 4100
+// bf16 12.1 / 9.5). Greedy rows only stream: about 1024 blocks each, from 5000 on (1 row of 2049 bf16 3.6 / 8.8,
+// 64 of 32000 6.0 / 11.4, 1 of 128256 22.3 / 8.4), and one wave merges them.
+int gumbel_segs(int64_t rows, int64_t nblk, bool greedy) {
+    if (nblk < (greedy ? 5000 : 400)) return 1;
+    const int64_t g = std::min<int64_t>(256 / rows, nblk / (greedy ? 1024 : 128));
     return int(std::min<int64_t>(std::max<int64_t>(g, 1), 64));
 }
 
@@ -160,7 +164,7 @@ extern "C" int nt_hip_rl_sample_gumbel(const NtRlGumbelArgs *a) {
     p.col = chacha_columns(p.key);
     hipStream_t s = ctx().stream;
     const int64_t nblk = V / 8 + 2;
-    p.segs = gumbel_segs(rows, nblk);
+    p.segs = gumbel_segs(rows, nblk, greedy);
     p.rec = nullptr;
     if (p.segs > 1) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
