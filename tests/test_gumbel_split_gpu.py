@@ -38,9 +38,10 @@ def test_tokens_at_the_edges_of_segments(rows, V, tau, mask, pre):
     keep = (rng.random((rows, V)) < 0.4).astype(np.uint8)
     keep[:, V // 2] = 1
     kw = {"keep": keep} if mask == "u8" else ({"addmask": np.where(keep, 0, -np.inf).astype(F)} if mask == "f32" else {})
-    dev, cpu = both(x, tau, 7 + rows, pre_u32=pre, **kw)
-    # (one token in 1000 may differ, two sums rounding apart; rows here are few)
-    assert np.count_nonzero(dev != cpu) <= (0 if tau == 0.0 else max(1, rows // 100))
+    # (streams enough for some 60 rows; the two sides' f64 logarithms, rounded to f32, part once in 1e8 draws)
+    for root in range(1 if tau == 0.0 else -(-60 // rows)):
+        dev, cpu = both(x, tau, 7 + rows + 1000 * root, pre_u32=pre, **kw)
+        np.testing.assert_array_equal(dev, cpu)
 
 
 def test_what_decides_a_row_lies_in_one_segment():
