@@ -23,7 +23,7 @@
 // A half product (GpuBackend::matmul_half; HALF) takes the same path: panels of 64 k rounded to bf16 on
 // their way into LDS, 16 k per v_mfma_f32_32x32x16_bf16, one accumulator over the whole of k.
 // Against the kernel before it, whose loads were branches between whole, unaligned and last panels:
-// 1024^3 24.2 -> 12.6 us, 247 x 525 x 914 39.9 -> 9.1, 300 x 3000 x 3000 391 -> 38.7, 2048^3 59.1 -> 38.4.
+// 1024^3 24.2 -> 12.6 us, 247 x 525 x 914 39.9 -> 9.1, 300 x 3000 x 3000 391 -> 38.7, 2048^3 59.1 -> 35.7.
 //
 // Workgroups are renumbered so that each of the 8 XCDs (which the hardware deals consecutive
 // workgroups to in turn) works on a contiguous run of tiles, whose A panels then stay in that
@@ -553,10 +553,10 @@ int tile_side(int64_t batches, int64_t m, int64_t n, int64_t least) {
     return big >= least && small > 2 * big ? 128 : 64;
 }
 
-template <bool HALF, bool SPLIT>
+template <bool HALF>
 int launch_tile(int tile, const MatmulP &p, hipStream_t s) {
-    if (tile == 128) return launch_matmul<HALF, Tile128, SPLIT>(p, s);
-    return launch_matmul<HALF, Tile64, SPLIT>(p, s);
+    if (tile == 128) return launch_matmul<HALF, Tile128, false>(p, s);
+    return launch_matmul<HALF, Tile64, false>(p, s);
 }
 
 }  // namespace
@@ -636,11 +636,11 @@ int nt_hip_matmul(const float *a, const NtLayout *al, const float *b, const NtLa
     std::unique_lock<std::mutex> lk;
     if (int rc = enter(&lk)) return rc;
     hipStream_t st = ctx().stream;
-    if (splits == 1) return launch_tile<false, false>(T, p, st);
+    if (splits == 1) return launch_tile<false>(T, p, st);
     void *sl = nullptr;
     if (int rc = scratch_alloc(size_t(nkc) * size_t(p.outputs) * sizeof(float), &sl)) return rc;
     p.slices = static_cast<float *>(sl);
-    int rc = launch_tile<false, true>(T, p, st);
+    int rc = launch_matmul<false, Tile64, true>(p, st);  // (fewer than 256 tiles: the 64 ones)
     if (!rc) {
         const int64_t fb = std::min<int64_t>((p.outputs + kMmThreads - 1) / kMmThreads, 4096);
         hipLaunchKernelGGL(k_fold, dim3(unsigned(fb)), dim3(kMmThreads), 0, st, p.slices, p.outputs, int(nkc), out);
@@ -736,7 +736,7 @@ int nt_hip_matmul_half(const float *a, const NtLayout *al, const float *b, const
     if (p.blocks > int64_t(0x7fffffff)) return fail(NT_E_ARG, "matmul_half: too many output tiles");
     std::unique_lock<std::mutex> lk;
     if (int rc = enter(&lk)) return rc;
-    return launch_tile<true, false>(T, p, ctx().stream);
+    return launch_tile<true>(T, p, ctx().stream);
 }
 
 int nt_hip_half_gemm_key(char *buf, size_t cap) {
