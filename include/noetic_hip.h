@@ -12,8 +12,10 @@
  *    ready after nt_hip_sync() or a download.
  *  - Every device entry point is serialised by one process-wide mutex (the reference's
  *    `CTX: OnceLock<Mutex<Ctx>>`, src/tensor/cuda/backend.rs:104,148-159).
- *  - Kernels use no atomics and reduce in a fixed order, so a rerun on the same inputs is
- *    bit-identical (the reference's determinism contract, src/nn/tests/gpu/rl.rs:125-128).
+ *  - Kernels reduce in a fixed order (atomics only where their order cannot reach a result), so a
+ *    rerun on the same inputs is bit-identical (the reference's determinism contract,
+ *    src/nn/tests/gpu/rl.rs:125-128). A row's scores have the same bits whatever rows are scored
+ *    with it, eagerly or under stream capture.
  *
  * A Rust caller binds these with a hand-written `extern "C"` block, the reference's FFI style
  * (src/tensor/cuda/ffi.rs:30-117), from optional GpuBackend methods.
@@ -99,7 +101,8 @@ int nt_hip_platform_details(char *buf, size_t cap);
  * work queued on the library stream after the call. nt_hip_free only records the pointer and
  * returns at once (the reference's Mem drop, src/tensor/cuda/backend.rs:35-45); the next entry
  * point keeps it for a later allocation of its size class (bounded; everything runs on the one
- * stream) or frees it on the stream, after the work queued before the release. */
+ * stream) or frees it on the stream, after the work queued before the release. Memory allocated
+ * before a stream capture and released during it stays allocated: the graph may use it. */
 int nt_hip_alloc(size_t bytes, void **out);
 int nt_hip_free(void *ptr);
 int nt_hip_upload(void *dst, const void *src, size_t bytes);   /* host -> device, synchronous */
@@ -311,7 +314,7 @@ typedef struct NtRlScoreArgs {
     float *entropy;           /* [rows] out or NULL */
     uint8_t *status;          /* [rows] out or NULL: NT_ROW_* of the policy row */
     /* The row's log-sum-exp, for nt_hip_rl_score_backward: lse = lse_base + lse_rest with
-     * lse_base a finite point at most 5 ln 2 below the maximum of the tempered logits and
+     * lse_base the maximum of the tempered logits and
      * lse_rest = ln sum exp(z - lse_base); both NaN on a refused row. Any of the four may be
      * NULL. */
     float *lse_base;          /* [rows] out or NULL (policy) */
